@@ -32,6 +32,7 @@
 // streaming pass over B on v_mfma_f32_16x16x4_f32); conv2d with
 // C*KH*KW <= 32 runs conv2d_direct_kernel.
 #include "common.h"
+#include "gemm_split.h"
 #include "row_softmax.h"
 
 #include <algorithm>
@@ -3246,19 +3247,20 @@ GemmArgs sgemm_args(const float *A, const float *B, float *C, int64_t M, int64_t
 
 // The kernels camel_hip_sgemm runs for a problem, and the bytes of split-K
 // partial sums they need (0 when nothing is split).
-enum class SgemmPath { Thin, Skinny, Tiles };
+enum class SgemmPath { Thin, Skinny, Split, Tiles };
 struct SgemmPlan {
     SgemmPath path;
     Cfg cfg;
     int splits;
     bool avec, bvec, atrans;
     size_t partial_bytes;
+    SplitPlan split;
 };
 
 // atrans: A is given transposed (CAMEL_GEMM_A_T); only the tile kernel has
 // the transposed loaders, so the thin and skinny kernels are not used.
 SgemmPlan plan_sgemm(const GemmArgs &g, bool atrans) {
-    SgemmPlan p{SgemmPath::Tiles, Cfg::Big, 1, false, false, atrans, 0};
+    SgemmPlan p{SgemmPath::Tiles, Cfg::Big, 1, false, false, atrans, 0, {}};
     if (!atrans && thin_eligible(g.M, g.N, g.K)) {
         p.path = SgemmPath::Thin;
         return p;
@@ -3272,6 +3274,14 @@ SgemmPlan plan_sgemm(const GemmArgs &g, bool atrans) {
     p.bvec = (g.N % 4 == 0) && ((uintptr_t)g.B % 16 == 0);
     int bk = 0;
     const int cus = device_cu_count();
+    if (g.M > 32) {
+        p.split = split_gemm_plan(g.M, g.N, g.K, atrans || !p.avec || !p.bvec, g.lda, g.ldb, cus);
+        if (p.split.tile != SplitTile::None) {
+            p.path = SgemmPath::Split;
+            p.partial_bytes = p.split.partial_bytes;
+            return p;
+        }
+    }
     choose(g.M, g.N, g.K, cus, p.cfg, p.splits, bk);
     if (p.cfg == Cfg::Mid && !atrans && p.avec && p.bvec && tiles_of<TileMid>(g.M, g.N) < 2 * cus)
         p.cfg = Cfg::MidK;
@@ -3304,6 +3314,23 @@ int run_sgemm(const GemmArgs &g, const SgemmPlan &p) {
         return launch_thin(g.A, g.B, g.C, g.M, g.N, g.K, g.bias, g.flags);
     case SgemmPath::Skinny:
         return launch_skinny(g.A, g.B, g.C, g.M, g.N, g.K, g.bias, g.flags);
+    case SgemmPath::Split: {
+        float *partial = nullptr;
+        if (p.partial_bytes) CAMEL_RETURN_IF(partial_buffer(p.partial_bytes, &partial));
+        SplitGemm s{};
+        s.A = g.A;
+        s.B = g.B;
+        s.C = g.C;
+        s.bias = g.bias;
+        s.M = g.M;
+        s.N = g.N;
+        s.K = g.K;
+        s.lda = g.lda;
+        s.ldb = g.ldb;
+        s.ldc = g.ldc;
+        s.flags = g.flags;
+        return split_gemm(s, p.atrans, p.split, partial);
+    }
     default:
         break;
     }
@@ -3410,6 +3437,11 @@ int camel_hip_dense_head(const float *x, const float *w1, const float *b1, const
         choose(M, N1, K1, device_cu_count(), cfg, splits, bk);
     const bool avec = (K1 % 4 == 0) && ((uintptr_t)x % 16 == 0);
     const bool bvec = (N1 % 4 == 0) && ((uintptr_t)w1 % 16 == 0);
+    // A first layer that camel_hip_sgemm gives to the split kernels runs as
+    // that call, and the head after it.
+    if (cfg != Cfg::Skinny &&
+        plan_sgemm(sgemm_args(x, w1, nullptr, M, N1, K1, b1, flags1), false).path == SgemmPath::Split)
+        cfg = Cfg::Skinny;
     if (cfg == Cfg::Small && splits <= 1 && avec && bvec && M % TileSmall::BM == 0 &&
         N1 % TileSmall::BN == 0 && N1 <= (int64_t)HEAD_MAX_N2 * TileSmall::BN &&
         N2 <= HEAD_MAX_N2 && M <= INT32_MAX / HEAD_MAX_N2) {
