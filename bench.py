@@ -696,7 +696,7 @@ def main() -> int:
         r = wl_conv(s_steps, s_warm)
         suite["conv2d_3x3"] = {"value": round(r["flop"] / (r["ms"] * 1e-3) / 1e9, 1),
                                "unit": "GFLOP/s", "ms": round(r["ms"], 4),
-                               "roofline": roofline_mfma(r["flop"], r["ms"], "conv2d")}
+                               "roofline": roofline_split(r["flop"], r["ms"], "conv2d")}
         cpu_jobs.append(("conv2d_3x3", lambda x=r["x"], w=r["w"], b=r["b"]:
                          cpu_baseline_conv(x, w, b, images=2)))
         r = wl_cnn(s_steps, s_warm)

@@ -3081,6 +3081,54 @@ int conv2d_gather(const float *x, const float *w, const float *bias, float *y, i
     return ok();
 }
 
+// True when conv2d runs on the split-operand kernels.  The first layers of an
+// image CNN that conv_pair_pool_kernel serves keep its fp32 MFMA sequence.
+bool conv_on_split(int64_t N, int64_t C, int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW,
+                   int64_t stride, int64_t pad) {
+    const bool pair_layer = C == CP_C1 && KH == 3 && KW == 3 && stride == 1 && pad == 0 && Co % 64 == 0;
+    return !pair_layer && split_conv_serves(N, C, H, W, Co, KH, KW, pad);
+}
+
+// conv2d on the split-operand kernels: x in any layout (NHWC and NCHW4 with
+// C % 4 == 0 and 16-byte alignment), y NCHW, NCHW4 (flags) or pooled.
+int conv2d_split(const float *x, const float *w, const float *bias, float *y, int64_t N, int64_t C,
+                 int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW, int64_t stride,
+                 int64_t pad, int64_t OH, int64_t OW, int flags, Layout x_layout, bool pool,
+                 bool w_packed) {
+    SplitConv c{};
+    c.C = (int)C;
+    c.H = (int)H;
+    c.W = (int)W;
+    c.KH = (int)KH;
+    c.KW = (int)KW;
+    c.stride = (int)stride;
+    c.pad = (int)pad;
+    c.P = (int)(OH * OW);
+    c.OW = (int)OW;
+    c.PW = (int)(OW / 2);
+    c.PP = (int)((OH / 2) * (OW / 2));
+    c.CHW = (int)(C * H * W);
+    c.HW = (int)(H * W);
+    c.pxs = x_layout == L_NHWC ? (int)C : x_layout == L_NCHW4 ? 4 : 1;
+    c.cqs = x_layout == L_NHWC ? 4 : (int)(4 * H * W);
+    c.bytes = (uint32_t)((N * C * H * W + pad * (W + 1) * c.pxs) * (int64_t)sizeof(float));
+    c.w_packed = w_packed;
+    SplitGemm g{};
+    g.A = w;
+    g.B = x;
+    g.C = y;
+    g.bias = bias;
+    g.M = (int)Co;
+    g.N = (int)(N * OH * OW);
+    g.K = (int)((C + 7) / 8 * 8 * KH * KW);
+    g.flags = flags;
+    Scratch ws;
+    const SplitConvPlan plan = split_conv_plan(g, c, pool, device_cu_count());
+    CAMEL_RETURN_IF(ws.alloc(plan.weight_bytes + plan.partial_bytes));
+    CAMEL_RETURN_IF(split_conv(g, c, x_layout != L_NCHW, pool, plan, ws.p));
+    return ok();
+}
+
 // Shared argument checks of the conv2d entry points.
 int conv_check(const float *x, const float *w, const float *bias, const float *y, int64_t N,
                int64_t C, int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW, int64_t stride,
@@ -3151,7 +3199,11 @@ int conv2d_run(const float *x, const float *w, const float *bias, float *y, int6
         flags &= ~CAMEL_CONV_W_PACKED;
     }
     // out_flags: the epilogue flags, plus CAMEL_CONV_Y_NCHW4 for an NCHW4 out
+    const bool split = conv_on_split(N, C, H, W, Co, KH, KW, stride, pad);
     auto nhwc_gemm = [&](float *out, bool pooled, int out_flags) -> int {
+        if (split)
+            return conv2d_split(x, w, bias, out, N, C, H, W, Co, KH, KW, stride, pad, OH, OW, out_flags, xl,
+                                pooled, w_packed);
         const bool k32 = C % 32 == 0;
         if (Co > 64)
             return k32 ? conv2d_nhwc<TileConv>(x, w, bias, out, N, C, H, W, Co, KH, KW, stride, pad, OH,
@@ -3200,6 +3252,9 @@ int conv2d_run(const float *x, const float *w, const float *bias, float *y, int6
         if (direct)
             CAMEL_RETURN_IF(conv2d_direct(xs, w, bias, out, N, C, H, W, Co, KH, KW, stride, pad, OH, OW,
                                           epi, out == y ? yl : L_NCHW));
+        else if (split)
+            CAMEL_RETURN_IF(conv2d_split(xs, w, bias, out, N, C, H, W, Co, KH, KW, stride, pad, OH, OW, epi,
+                                         L_NCHW, false, false));
         else
             CAMEL_RETURN_IF(conv2d_gather(xs, w, bias, out, N, C, H, W, Co, KH, KW, stride, pad, OH, OW,
                                           epi));

@@ -20,6 +20,27 @@ struct SplitGemm {
     int flags;       // CAMEL_EPI_*, conv: CAMEL_CONV_Y_NCHW4
 };
 
+// A convolution as that GEMM: M = output channels, N = pixels (batch OH OW, or
+// 4 per pool window), K = taps x channels padded to a multiple of 8 (see `unit`).
+struct SplitConv {
+    typedef uint32_t chunk __attribute__((ext_vector_type(4)));
+    // set by split_conv, with kpad, unit, taps, shift, the multipliers, patch
+    // and per_image
+    const chunk *w_split;
+    int kpad;
+    int C, H, W, KH, KW, stride, pad;
+    int unit, taps; // K as runs of `unit` channels of one of the taps
+    int P, OW;    // output pixels per image, width
+    int PW, PP;   // pool windows per row, per image (pooled)
+    int CHW, HW;  // input elements per image, per plane
+    int pxs, cqs; // distance of pixels and (quads) of channel quads
+    int shift;    // elements before x that the first window reaches back
+    uint32_t bytes;          // of x and the shift before it
+    uint32_t mul_unit, mul_kw, mul_taps; // floor(n / d) = n mul >> 32 for n < 65536
+    int patch, per_image;    // positions of a patch (0: not that kernel), tiles per image
+    int w_packed;            // weights [Co][KH][KW][C], else [Co][C][KH][KW]
+};
+
 // How the split kernels run a GEMM: the tile and the K splits.
 enum class SplitTile { None, T256, T128 };
 struct SplitPlan {
@@ -35,5 +56,22 @@ SplitPlan split_gemm_plan(int64_t M, int64_t N, int64_t K, bool unaligned, int64
                           int cus);
 // Runs it on the library stream; `partial`: plan.partial_bytes of scratch.
 int split_gemm(SplitGemm g, bool a_trans, const SplitPlan &plan, float *partial);
+
+// True when split_conv serves the geometry (either layout).
+bool split_conv_serves(int64_t N, int64_t C, int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW,
+                       int64_t pad);
+// The kernel and K splits of a convolution and its scratch: the split weights,
+// then the partial sums.
+struct SplitConvPlan {
+    int blocked = 0, patch = 0;
+    int per_image = 0;
+    int splits = 1;
+    size_t weight_bytes = 0, partial_bytes = 0;
+};
+// (g.N: the pixels of the unpooled output, here and below.)
+SplitConvPlan split_conv_plan(const SplitGemm &g, const SplitConv &c, bool pool, int cus);
+// Runs it (`quads`: x in NHWC or NCHW4, else NCHW; `pool`: the 2x2 pooled
+// output); `scratch`: weight_bytes + partial_bytes.
+int split_conv(SplitGemm g, SplitConv c, bool quads, bool pool, const SplitConvPlan &plan, void *scratch);
 
 } // namespace camel_hip

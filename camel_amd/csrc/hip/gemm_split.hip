@@ -19,9 +19,9 @@
 // Operands outside the exact range, tile by tile: the converting lanes keep
 // the smallest nonzero |hi| (two packed 16-bit operations per pair), and a
 // value that is infinite, NaN or beyond the bf16 maximum makes its outputs
-// non-finite (its mid part is).  A tile that saw |x| < 2^-100 or holds a
-// non-finite sum is computed again in fp32 MFMA, so special values and the
-// ends of the range give what they give in fp32.
+// non-finite (its mid part is).  A tile that saw |x| < 2^-100 is computed again
+// in fp32 MFMA, and so are the non-finite sums of any other tile: special
+// values and the ends of the range give what they give in fp32.
 //
 // Tile: waves as WM x WN, each FM x FN blocks of 16 x 16; A goes from global
 // memory straight into the registers of the waves that multiply it (lane (r,
@@ -65,24 +65,30 @@ __device__ __forceinline__ float upper(float x) {
     return __uint_as_float(__float_as_uint(x) & 0xffff0000u);
 }
 
-// f[0..7] -> three chunks of 8 bf16 (hi, mid, lo); tiny: running minimum of
-// 2 |hi| - 1.  (v_dot2_f32_bf16 with a -1 forms x - hi in one operation
+// tiny = min(tiny, 2 |h| - 1) over a pair of bf16.
+__device__ __forceinline__ void note_tiny(uint32_t h, us2 &tiny) {
+    us2 twice;
+    asm("v_pk_mad_u16 %0, %1, 2, -1 op_sel_hi:[1,0,0]" : "=v"(twice) : "v"(h));
+    tiny = __builtin_elementwise_min(tiny, twice);
+}
+
+// Pair c of f[0..7] (split8: all four) into three chunks of 8 bf16 (hi, mid,
+// lo); tiny: running minimum of 2 |hi| - 1.  (v_dot2_f32_bf16 with a -1 forms x - hi in one operation
 // instead of two, but its results may not be read for 3 wait states: 4096^3
 // 557 -> 578 us.)
+__device__ __forceinline__ void split_pair(const float *f, int c, u4 *out, us2 &tiny) {
+    float x0 = f[2 * c], x1 = f[2 * c + 1];
+    const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){x0, x1}, bf2));
+    note_tiny(h, tiny);
+    x0 = x0 - __uint_as_float(h << 16);
+    x1 = x1 - __uint_as_float(h & 0xffff0000u);
+    out[0][c] = h;
+    out[1][c] = upper_pair(x0, x1);
+    out[2][c] = upper_pair(x0 - upper(x0), x1 - upper(x1));
+}
 __device__ __forceinline__ void split8(const float *f, u4 *out, us2 &tiny) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        float x0 = f[2 * c], x1 = f[2 * c + 1];
-        const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){x0, x1}, bf2));
-        us2 twice;
-        asm("v_pk_mad_u16 %0, %1, 2, -1 op_sel_hi:[1,0,0]" : "=v"(twice) : "v"(h));
-        tiny = __builtin_elementwise_min(tiny, twice);
-        x0 = x0 - __uint_as_float(h << 16);
-        x1 = x1 - __uint_as_float(h & 0xffff0000u);
-        out[0][c] = h;
-        out[1][c] = upper_pair(x0, x1);
-        out[2][c] = upper_pair(x0 - upper(x0), x1 - upper(x1));
-    }
+    for (int c = 0; c < 4; ++c) split_pair(f, c, out, tiny);
 }
 
 // WM x WN waves of FM x FN blocks; WK groups of them take alternate stages of
@@ -112,14 +118,19 @@ __device__ __forceinline__ void split_tile_of(int id, int tiles_m, int tiles_n, 
     tn = in_group / gsize;
 }
 
+// Where the A operand comes from: row-major fp32, transposed fp32, or already
+// split ([stage][16-row block][part][64 lanes] chunks, the conv weights).
+enum ASource { A_ROWS, A_COLS, A_SPLIT };
+enum Output { OUT_MATRIX, OUT_CONV, OUT_POOL };
+
 // B as a row-major matrix: lane = column, octet o of a stage = rows 8 o .. +7,
 // 256 contiguous bytes of a row per load.
 template <class T> struct MatrixB {
     const float *base;
     int ld;
     uint32_t off[T::B_IT];
-    __device__ __forceinline__ MatrixB(const SplitGemm &g) : base(g.B), ld(g.ldb) {}
-    __device__ __forceinline__ void column(const SplitGemm &g, int i, int n) {
+    __device__ __forceinline__ MatrixB(const SplitGemm &g, const SplitConv &) : base(g.B), ld(g.ldb) {}
+    __device__ __forceinline__ void column(const SplitGemm &g, const SplitConv &, int i, int n) {
         off[i] = (uint32_t)min(n, g.N - 1) * 4u;
     }
     // 8 rows from k (all inside [0, K))
@@ -139,10 +150,139 @@ template <class T> struct MatrixB {
                              : *reinterpret_cast<const float *>(
                                    reinterpret_cast<const char *>(base + (size_t)(k + j) * ld) + off[i]);
     }
-    __device__ __forceinline__ static float at(const SplitGemm &g, int k, int n) {
+    __device__ __forceinline__ static float at(const SplitGemm &g, const SplitConv &, int k, int n) {
         return g.B[(size_t)k * g.ldb + n];
     }
 };
+
+// Image, row and column of GEMM column n of a convolution: pixels in order, or
+// (POOL) 4 per window of the 2x2 pool, ((0,0), (0,1), (1,0), (1,1)).
+template <bool POOL>
+__device__ __forceinline__ void conv_pixel(const SplitConv &c, int n, int &img, int &oh, int &ow) {
+    if constexpr (POOL) {
+        img = n / (4 * c.PP);
+        const int r = n - img * 4 * c.PP, win = r >> 2, d = r & 3, ph = win / c.PW;
+        oh = 2 * ph + (d >> 1);
+        ow = 2 * (win - ph * c.PW) + (d & 1);
+    } else {
+        img = n / c.P;
+        const int r = n - img * c.P;
+        oh = r / c.OW;
+        ow = r - oh * c.OW;
+    }
+}
+
+// Tap and channel of k: runs of `unit` channels of one tap, tap after tap, then
+// the next `unit` channels (unit: all channels padded to 8, or 32).
+__device__ __forceinline__ void conv_k(const SplitConv &c, int k, int &tap, int &ch) {
+    const int run = k / c.unit, blk = run / c.taps;
+    tap = run - blk * c.taps;
+    ch = blk * c.unit + k - run * c.unit;
+}
+
+// Element (k, n) of the im2col matrix.
+template <bool QUADS, bool POOL>
+__device__ __forceinline__ float conv_input(const SplitGemm &g, const SplitConv &c, int k, int n) {
+    int tap, ch;
+    conv_k(c, k, tap, ch);
+    const int kh = tap / c.KW, kw = tap - kh * c.KW;
+    int img, oh, ow;
+    conv_pixel<POOL>(c, n, img, oh, ow);
+    const int ih = oh * c.stride - c.pad + kh, iw = ow * c.stride - c.pad + kw;
+    if (ch >= c.C || (unsigned)ih >= (unsigned)c.H || (unsigned)iw >= (unsigned)c.W) return 0.f;
+    const size_t px = (size_t)img * c.CHW + (size_t)(ih * c.W + iw) * c.pxs;
+    return QUADS ? g.B[px + (size_t)(ch >> 2) * c.cqs + (ch & 3)] : g.B[px + (size_t)ch * c.HW];
+}
+
+// B as the im2col matrix of a convolution, K ordered as conv_k: an octet is 8 channels of one tap, the
+// same for a whole wave, so its offset is scalar, and a lane's pixel gives the
+// vector offset.  Buffer loads: a lane whose tap lies in the padding (a bit
+// per tap, decoded once) or a channel past C takes an offset past the end of
+// the buffer, which reads zero.  QUADS: channel quads 16 bytes apart in
+// memory or side by side (NHWC, NCHW4), two 16-byte loads; else 8 planes, 256
+// contiguous bytes of one each (for a stride of 1).
+constexpr uint32_t NO_ELEMENT = 1u << 31; // buffers and scalar offsets stay below 2^31 bytes
+template <class T, bool QUADS, bool POOL> struct ConvB {
+    const SplitConv &c;
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t off[T::B_IT], taps[T::B_IT];
+    __device__ __forceinline__ ConvB(const SplitGemm &g, const SplitConv &cv) : c(cv) {
+        // offsets count from `shift` elements before x, so that the window of
+        // the first pixel starts at 0
+        rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(g.B - c.shift), 0, c.bytes, 0x00027000);
+    }
+    __device__ __forceinline__ void column(const SplitGemm &g, const SplitConv &, int i, int n) {
+        int img, oh, ow;
+        conv_pixel<POOL>(c, min(n, g.N - 1), img, oh, ow);
+        const int ih = oh * c.stride - c.pad, iw = ow * c.stride - c.pad;
+        off[i] = (uint32_t)(img * c.CHW + (ih * c.W + iw) * c.pxs + c.shift) * 4u;
+        uint32_t m = 0;
+        for (int kh = 0, t = 0; kh < c.KH; ++kh)
+            for (int kw = 0; kw < c.KW; ++kw, ++t)
+                m |= ((unsigned)(ih + kh) < (unsigned)c.H && (unsigned)(iw + kw) < (unsigned)c.W) ? 1u << t : 0u;
+        taps[i] = m;
+    }
+    __device__ __forceinline__ void load(int i, int k, float *f) const {
+        const int run = (int)__umulhi((uint32_t)k, c.mul_unit), blk = (int)__umulhi((uint32_t)run, c.mul_taps);
+        const int tap = run - blk * c.taps, c0 = blk * c.unit + k - run * c.unit;
+        const int kh = (int)__umulhi((uint32_t)tap, c.mul_kw), kw = tap - kh * c.KW;
+        const uint32_t v = (taps[i] >> tap) & 1 ? off[i] : NO_ELEMENT;
+        const uint32_t s = (uint32_t)((kh * c.W + kw) * c.pxs) * 4u;
+        if constexpr (QUADS) {
+            const uint32_t so = s + (uint32_t)((c0 >> 2) * c.cqs) * 4u;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const u4 q = __builtin_amdgcn_raw_buffer_load_b128(rsrc, c0 + 4 * h < c.C ? v : NO_ELEMENT,
+                                                                   so + (uint32_t)(h * c.cqs) * 4u, 0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) f[4 * h + j] = __uint_as_float(q[j]);
+            }
+        } else {
+            uint32_t so = s + (uint32_t)(c0 * c.HW) * 4u;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                f[j] = __uint_as_float(
+                    __builtin_amdgcn_raw_buffer_load_b32(rsrc, c0 + j < c.C ? v : NO_ELEMENT, so, 0));
+                so += (uint32_t)c.HW * 4u;
+            }
+        }
+    }
+    // an octet is wholly below 0 or not at all
+    __device__ __forceinline__ void load_ragged(int i, int k, float *f) const {
+        load(i, max(k, 0), f);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[j] = k < 0 ? 0.f : f[j];
+    }
+    __device__ __forceinline__ static float at(const SplitGemm &g, const SplitConv &c, int k, int n) {
+        return conv_input<QUADS, POOL>(g, c, k, n);
+    }
+};
+
+// Weight (row, k) of a convolution.
+__device__ __forceinline__ float conv_weight(const SplitGemm &g, const SplitConv &c, int row, int k) {
+    int tap, ch;
+    conv_k(c, k, tap, ch);
+    if (ch >= c.C) return 0.f;
+    return g.A[c.w_packed ? ((size_t)row * c.taps + tap) * c.C + ch : ((size_t)row * c.C + ch) * c.taps + tap];
+}
+
+// The weights of a convolution as the MFMA operand, split: stage blockIdx.x,
+// 16-row block blockIdx.y, lane (r16, oct) its 8 k.  Rows past Co repeat the
+// last one.
+__global__ __launch_bounds__(64) void split_weights_kernel(SplitGemm g, SplitConv c, u4 *dst) {
+    const int lane = threadIdx.x, stage = blockIdx.x, blk = blockIdx.y;
+    const int kpad = gridDim.x * BK - g.K;
+    const int row = min(16 * blk + (lane & 15), g.M - 1), k0 = stage * BK - kpad + 8 * (lane >> 4);
+    float f[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = k0 < 0 ? 0.f : conv_weight(g, c, row, k0 + j);
+    u4 out[3];
+    us2 tiny = {0xffff, 0xffff};
+    split8(f, out, tiny);
+    u4 *d = dst + ((size_t)stage * gridDim.y + blk) * 192 + lane;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) d[64 * q] = out[q];
+}
 
 // Lane (r16, oct) holds columns nw + 16 j + 4 oct .. +3 of rows mw + 16 i (mw
 // and nw include the lane): bias and relu, or the split's partial sums.
@@ -181,9 +321,335 @@ __device__ __forceinline__ void store_matrix(const SplitGemm &g, f4 (*acc)[FN], 
     }
 }
 
-template <class T, bool AT>
-__global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g) {
-    using BSrc = MatrixB<T>;
+// Image and place in it of GEMM column n of a convolution's output (per = P, or
+// 4 PP columns per image when pooled).
+struct ConvColumn {
+    int img, p;
+    __device__ __forceinline__ ConvColumn(int n, int per) : img(n / per), p(n - img * per) {}
+    __device__ __forceinline__ void advance(int by, int per) {
+        for (p += by; p >= per; p -= per) ++img;
+    }
+};
+
+// 4 columns (from n, at col) of output channel `row` of a convolution: bias and
+// relu, then NCHW, NCHW4, or (POOL: the columns are a window) the window's
+// maximum by the pool's rule, first then strict '>'.
+template <bool POOL>
+__device__ __forceinline__ void store_conv_quad(const SplitGemm &g, const SplitConv &c, f4 x, int row, int n,
+                                                ConvColumn col, float bias) {
+    const bool q4 = (g.flags & CAMEL_CONV_Y_NCHW4) != 0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        if (g.flags & CAMEL_EPI_BIAS) x[v] = x[v] + bias;
+        if (g.flags & CAMEL_EPI_RELU) x[v] = relu_idiom(x[v]);
+    }
+    if constexpr (POOL) {
+        float mx = x[0];
+#pragma unroll
+        for (int v = 1; v < 4; ++v)
+            if (x[v] > mx) mx = x[v];
+        g.C[((size_t)col.img * g.M + row) * c.PP + (col.p >> 2)] = mx;
+        return;
+    }
+    if (!q4 && col.p + 3 < c.P) {
+        *reinterpret_cast<f4u *>(g.C + ((size_t)col.img * g.M + row) * c.P + col.p) = x;
+        return;
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        if (n + v < g.N)
+            g.C[q4 ? (size_t)col.img * g.M * c.P + (size_t)(row & ~3) * c.P + 4 * (size_t)col.p + (row & 3)
+                   : ((size_t)col.img * g.M + row) * c.P + col.p] = x[v];
+        col.advance(1, c.P);
+    }
+}
+
+// The lanes' results (as store_matrix) of a convolution, rows = output
+// channels; or the split's partial sums.
+template <int FM, int FN, bool POOL>
+__device__ __forceinline__ void store_conv(const SplitGemm &g, const SplitConv &c, f4 (*acc)[FN], int split,
+                                           int mw, int nw) {
+    if (g.partial) {
+        SplitGemm part = g;
+        part.flags = 0;
+        store_matrix<FM, FN>(part, acc, split, mw, nw);
+        return;
+    }
+    float bias[FM];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+        bias[i] = (g.flags & CAMEL_EPI_BIAS) ? g.bias[min(mw + 16 * i, g.M - 1)] : 0.f;
+    const int per = POOL ? 4 * c.PP : c.P;
+    ConvColumn col(nw, per);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        if (nw + 16 * j >= g.N) break;
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+            if (mw + 16 * i < g.M) store_conv_quad<POOL>(g, c, acc[i][j], mw + 16 * i, nw + 16 * j, col, bias[i]);
+        col.advance(16, per);
+    }
+}
+
+// The sums of a tile that the split cannot form: all of them where an operand
+// was below its range (flag bit TINY_SEEN), the non-finite ones otherwise, in
+// fp32 (v_mfma_f32_16x16x4_f32, the same result layout), 4 columns of blocks at
+// a time.  a(i, k), b(j, k): this lane's operand of block row i, column j.
+enum { TINY_SEEN = 1, NOT_FINITE = 2 };
+template <int FM, int FN, class A, class B>
+__device__ __forceinline__ void fp32_sums(f4 (*acc)[FN], int kbeg, int kend, bool all, int oct, A a, B b) {
+    static_assert(FN % 4 == 0, "columns in fours");
+    auto sums = [&](int j0, auto &y, int jy) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[i][jy + j] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int k0 = kbeg; k0 < kend; k0 += 4) {
+            const int k = k0 + oct;
+            float fa[FM], fb[4];
+#pragma unroll
+            for (int i = 0; i < FM; ++i) fa[i] = k < kend ? a(i, k) : 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) fb[j] = k < kend ? b(j0 + j, k) : 0.f;
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    y[i][jy + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j], fa[i], y[i][jy + j], 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int j0 = 0; j0 < FN; j0 += 4) {
+        if constexpr (FM * FN > 16) { // no registers for both: all of them
+            sums(j0, acc, j0);
+        } else {
+            f4 y[FM][4];
+            sums(j0, y, 0);
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (all || !(__builtin_fabsf(acc[i][j0 + j][v]) < INFINITY)) acc[i][j0 + j][v] = y[i][j][v];
+        }
+    }
+}
+
+// Stride-1 convolution with the input converted once per work-group instead
+// of once per tap: a tile's output pixels read a contiguous range of the
+// zero-padded image (position (img Hp + ih) Wp + iw; tap (kh, kw) adds kh Wp +
+// kw), at most PATCH positions.  For 32 channels at a time that range goes to
+// LDS as split chunks [part][octet][position]; all taps then multiply from it
+// with no conversion, store or barrier between them, and the next 32 channels'
+// loads are in flight meanwhile.  16 output pixels read 16 nearly always
+// consecutive positions, so the reads are free of bank conflicts.  Weights
+// come split, straight into registers, a tap ahead.
+// 64 x 64 x 56 x 56 -> 128 3x3: 286 us on the fp32 MFMA implicit GEMM, 206 with
+// the im2col loads above, 160 so (188 TFLOP/s; in-kernel 65% of the matrix
+// pipe's cycles, the rest the patch's conversion, tile ends and 3.1 rounds).
+template <int FM_, int FN_, int WM_, int WN_> struct PatchTile {
+    static constexpr int FM = FM_, FN = FN_, WM = WM_, WN = WN_;
+    static constexpr int BM = 16 * FM * WM, BN = 16 * FN * WN;
+    static constexpr int THREADS = 64 * WM * WN;
+    static_assert(WM * WN == 4, "a wave per octet loads the patch");
+};
+constexpr int PATCH = 320;               // positions: 60 KiB, two work-groups per CU
+constexpr int PATCH_IT = (PATCH + 63) / 64;
+
+template <class T, bool QUADS, bool POOL>
+__global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, SplitConv c) {
+    __shared__ u4 patch[12 * PATCH + 1];
+    uint32_t *const flag = reinterpret_cast<uint32_t *>(patch + 12 * PATCH);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / T::WN, wn = wave - wm * T::WN;
+    const int r16 = lane & 15, oct = lane >> 4;
+    const int per = POOL ? 4 * c.PP : c.P; // columns per image
+    const int tiles_m = (g.M + T::BM - 1) / T::BM, tiles_i = (per + T::BN - 1) / T::BN;
+    const int nt = gridDim.x; // tiles_m x (tiles of an image x images, or of all columns)
+    int bid = blockIdx.x;
+    if ((nt & 7) == 0) bid = (bid & 7) * (nt >> 3) + (bid >> 3);
+    const int tn = bid / tiles_m, tm = bid - tn * tiles_m;
+    const int m0 = tm * T::BM;
+    // columns n0 .. nend - 1 (a tile of its image, or of all)
+    const int n0 = c.per_image ? tn / tiles_i * per + tn % tiles_i * T::BN : tn * T::BN;
+    const int nend = c.per_image ? (tn / tiles_i + 1) * per : g.N;
+    const int Hp = c.H + 2 * c.pad, Wp = c.W + 2 * c.pad, taps = c.taps;
+    if (tid == 0) *flag = 0;
+    auto position = [&](int n) {
+        int img, oh, ow;
+        conv_pixel<POOL>(c, min(n, nend - 1), img, oh, ow);
+        return (img * Hp + oh) * Wp + ow;
+    };
+    // Columns past the tile's end repeat the last one.  (Pool order: a
+    // window's first column has the least position, but windows of one pool
+    // row come before the row below it, so the tile's least is column n0's.)
+    const int q0 = position(n0);
+
+    // This lane's patch items: position lane + 64 i, octet `wave`.
+    uint32_t off[PATCH_IT];
+    {
+        const int last = g.N / per * Hp * Wp; // positions of all images
+#pragma unroll
+        for (int i = 0; i < PATCH_IT; ++i) {
+            const int q = q0 + lane + 64 * i, row = q / Wp, iw = q - row * Wp - c.pad;
+            const int img = row / Hp, ih = row - img * Hp - c.pad;
+            const bool in = q < last && (unsigned)ih < (unsigned)c.H && (unsigned)iw < (unsigned)c.W;
+            off[i] = in ? (uint32_t)(img * c.CHW + (ih * c.W + iw) * c.pxs) * 4u : NO_ELEMENT;
+        }
+    }
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(g.B), 0, c.bytes, 0x00027000);
+    float raw[PATCH_IT][8];
+    auto load_patch = [&](int blk) {
+        const int c0 = blk * BK + 8 * wave;
+#pragma unroll
+        for (int i = 0; i < PATCH_IT; ++i) {
+            if (64 * i >= c.patch) break;
+            if constexpr (QUADS) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const u4 q = __builtin_amdgcn_raw_buffer_load_b128(
+                        rsrc, c0 + 4 * h < c.C ? off[i] : NO_ELEMENT, (uint32_t)(((c0 >> 2) + h) * c.cqs) * 4u, 0);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) raw[i][4 * h + j] = __uint_as_float(q[j]);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    raw[i][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                        rsrc, c0 + j < c.C ? off[i] : NO_ELEMENT, (uint32_t)((c0 + j) * c.HW) * 4u, 0));
+            }
+        }
+    };
+    us2 tiny = {0xffff, 0xffff};
+    auto store_patch = [&]() {
+#pragma unroll
+        for (int i = 0; i < PATCH_IT; ++i) {
+            if (64 * i >= c.patch) break;
+            u4 d[3];
+            split8(raw[i], d, tiny);
+            if (64 * i + lane < PATCH)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) patch[(q * 4 + wave) * PATCH + 64 * i + lane] = d[q];
+        }
+    };
+    // Operand chunks of the lane's columns: at[j] + tap offset.
+    int at[T::FN];
+#pragma unroll
+    for (int j = 0; j < T::FN; ++j)
+        at[j] = oct * PATCH + position(n0 + (wn * T::FN + j) * 16 + r16) - q0;
+    const int a_blocks = (g.M + 15) / 16;
+    const u4 *a_src[T::FM];
+#pragma unroll
+    for (int i = 0; i < T::FM; ++i)
+        a_src[i] = c.w_split + (size_t)min(m0 / 16 + wm * T::FM + i, a_blocks - 1) * 192 + lane;
+    const int blocks = (c.C + BK - 1) / BK, stages = blocks * taps;
+    u4 an[T::FM][3];
+    auto load_a = [&](int stage) { // past the end the last one again
+        const size_t o = (size_t)min(stage, stages - 1) * a_blocks * 192;
+#pragma unroll
+        for (int i = 0; i < T::FM; ++i)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) an[i][q] = a_src[i][o + 64 * q];
+    };
+    f4 acc[T::FM][T::FN];
+#pragma unroll
+    for (int i = 0; i < T::FM; ++i)
+#pragma unroll
+        for (int j = 0; j < T::FN; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    load_patch(0);
+    load_a(0);
+    bf8 b[2][3], a[T::FM][3];
+    f4 t[2][T::FM];
+    auto fetch = [&](int j, int tap_off, bf8 *d) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+            d[q] = __builtin_bit_cast(bf8, patch[q * 4 * PATCH + at[j] + tap_off]);
+    };
+    constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+    int stage = 0;
+    for (int blk = 0; blk < blocks; ++blk) {
+        if (blk > 0) __syncthreads(); // the block before is multiplied
+        store_patch();
+        __syncthreads();
+        if (blk + 1 < blocks) load_patch(blk + 1);
+        fetch(0, 0, b[0]);
+        int kw = 0, tap_off = 0;
+        for (int tap = 0; tap < taps; ++tap, ++stage) {
+#pragma unroll
+            for (int i = 0; i < T::FM; ++i)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    a[i][q] = __builtin_bit_cast(bf8, an[i][q]);
+                    if (q == 0)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) note_tiny(an[i][0][e], tiny);
+                }
+            load_a(stage + 1);
+            // next tap's offset (after the last one this tap's again)
+            int next_off = tap_off + 1;
+            if (++kw == c.KW) {
+                kw = 0;
+                next_off = tap_off + 1 + Wp - c.KW;
+            }
+            if (tap + 1 == taps) next_off = tap_off;
+#pragma unroll
+            for (int j = 0; j < T::FN; ++j) {
+                fetch((j + 1) % T::FN, j + 1 < T::FN ? tap_off : next_off, b[(j + 1) & 1]);
+#pragma unroll
+                for (int i = 0; i < T::FM; ++i) t[j & 1][i] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int p = 0; p < 6; ++p)
+#pragma unroll
+                    for (int i = 0; i < T::FM; ++i)
+                        t[j & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j & 1][PB[p]], a[i][PA[p]],
+                                                                              t[j & 1][i], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < T::FM; ++i)
+                    if (j > 0) acc[i][j - 1] += t[(j + 1) & 1][i];
+#pragma unroll
+                for (int r = 0; r < 6 * T::FM; ++r) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    if (r % T::FM == T::FM - 1 && r < 3 * T::FM) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    if (r >= T::FM) __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int i = 0; i < T::FM; ++i) acc[i][T::FN - 1] += t[(T::FN - 1) & 1][i];
+            tap_off = next_off;
+        }
+    }
+
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < T::FM; ++i)
+#pragma unroll
+        for (int j = 0; j < T::FN; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
+    if (bad) atomicOr(flag, (uint32_t)NOT_FINITE);
+    if (tiny.x < TINY || tiny.y < TINY) atomicOr(flag, (uint32_t)TINY_SEEN);
+    __syncthreads();
+    const int mw = m0 + wm * T::FM * 16 + r16, nw = n0 + wn * T::FN * 16;
+    if (*flag)
+        fp32_sums<T::FM, T::FN>(
+            acc, 0, g.K, *flag & TINY_SEEN, oct,
+            [&](int i, int k) { return conv_weight(g, c, min(mw + 16 * i, g.M - 1), k); },
+            [&](int j, int k) { return conv_input<QUADS, POOL>(g, c, k, min(nw + 16 * j + r16, nend - 1)); });
+    SplitGemm tile = g;
+    tile.N = nend;
+    tile.partial = nullptr;
+    store_conv<T::FM, T::FN, POOL>(tile, c, acc, 0, mw, nw + 4 * oct);
+}
+
+// (The conv kernels' first stage below k = 0 is stage 0 of the split weights.)
+template <class T, int ASRC, class BSrc, int OUT>
+__global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, SplitConv cv) {
+    constexpr bool AT = ASRC == A_COLS;
     __shared__ u4 smem[T::LDS + 1];
     uint32_t *const flag = reinterpret_cast<uint32_t *>(smem + T::LDS);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -211,41 +677,56 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g) 
 
     // Rows and columns past the problem repeat the last one (never stored).
     const int mw = m0 + wm * T::FM * 16 + r16;
-    const float *a_base = AT ? g.A : g.A + (size_t)m0 * g.lda;
+    const float *a_base = ASRC == A_ROWS ? g.A + (size_t)m0 * g.lda : g.A;
     uint32_t a_off[T::FM];
+    const int a_blocks = (g.M + 15) / 16; // A_SPLIT
 #pragma unroll
     for (int i = 0; i < T::FM; ++i) {
+        if constexpr (ASRC == A_SPLIT) {
+            a_off[i] = (uint32_t)min(m0 / 16 + wm * T::FM + i, a_blocks - 1) * 192u + lane;
+            continue;
+        }
         const int row = min(mw + 16 * i, g.M - 1);
         a_off[i] = AT ? (uint32_t)row * 4u + (uint32_t)(8 * oct) * (uint32_t)g.lda * 4u
                       : (uint32_t)(row - m0) * (uint32_t)g.lda * 4u + 32u * oct;
     }
-    auto load_a = [&](int k0, float (*f)[8]) {
+    // A's stage at k0: 8 fp32 values a block, or (A_SPLIT) its three chunks.
+    struct ARegs {
+        float f[ASRC == A_SPLIT ? 1 : T::FM][8];
+        u4 c[ASRC == A_SPLIT ? T::FM : 1][3];
+    };
+    auto load_a = [&](int k0, int i, ARegs &r) {
+        if constexpr (ASRC == A_SPLIT) {
+            const u4 *q = cv.w_split + (size_t)((k0 + cv.kpad) / BK) * a_blocks * 192 + a_off[i];
 #pragma unroll
-        for (int i = 0; i < T::FM; ++i) {
-            if constexpr (!AT) {
-                const char *q = reinterpret_cast<const char *>(a_base + k0) + a_off[i];
-                const f4 v0 = *reinterpret_cast<const f4u *>(q);
-                const f4 v1 = *reinterpret_cast<const f4u *>(q + 16);
+            for (int p = 0; p < 3; ++p) r.c[i][p] = q[64 * p];
+        } else if constexpr (!AT) {
+            const char *q = reinterpret_cast<const char *>(a_base + k0) + a_off[i];
+            const f4 v0 = *reinterpret_cast<const f4u *>(q);
+            const f4 v1 = *reinterpret_cast<const f4u *>(q + 16);
 #pragma unroll
-                for (int c = 0; c < 4; ++c) f[i][c] = v0[c], f[i][4 + c] = v1[c];
-            } else {
-                const char *q = reinterpret_cast<const char *>(a_base + (size_t)k0 * g.lda);
+            for (int c = 0; c < 4; ++c) r.f[i][c] = v0[c], r.f[i][4 + c] = v1[c];
+        } else {
+            const char *q = reinterpret_cast<const char *>(a_base + (size_t)k0 * g.lda);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    f[i][j] = *reinterpret_cast<const float *>(q + a_off[i]);
-                    q += (size_t)g.lda * sizeof(float);
-                }
+            for (int j = 0; j < 8; ++j) {
+                r.f[i][j] = *reinterpret_cast<const float *>(q + a_off[i]);
+                q += (size_t)g.lda * sizeof(float);
             }
         }
     };
-    BSrc bsrc(g);
+    auto load_all_a = [&](int k0, ARegs &r) {
+#pragma unroll
+        for (int i = 0; i < T::FM; ++i) load_a(k0, i, r);
+    };
+    BSrc bsrc(g, cv);
     int b_slot[T::B_IT], b_oct[T::B_IT];
 #pragma unroll
     for (int i = 0; i < T::B_IT; ++i) {
         const int wi = w + i * T::GW, c = (wi >> 2) * 64 + lane;
         b_oct[i] = wi & 3;
         b_slot[i] = b_oct[i] * T::BN + c;
-        bsrc.column(g, i, n0 + c);
+        bsrc.column(g, cv, i, n0 + c);
     }
     auto load_b = [&](int k0, float (*f)[8]) {
 #pragma unroll
@@ -262,11 +743,18 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g) 
         }
     };
     bf8 a[T::FM][3];
-    auto split_a = [&](float (*f)[8]) {
+    auto split_a = [&](const ARegs &r) {
 #pragma unroll
         for (int i = 0; i < T::FM; ++i) {
             u4 c[3];
-            split8(f[i], c, tiny);
+            if constexpr (ASRC == A_SPLIT) {
+#pragma unroll
+                for (int q = 0; q < 3; ++q) c[q] = r.c[i][q];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) note_tiny(c[0][q], tiny);
+            } else {
+                split8(r.f[i], c, tiny);
+            }
 #pragma unroll
             for (int q = 0; q < 3; ++q) a[i][q] = __builtin_bit_cast(bf8, c[q]);
         }
@@ -280,18 +768,20 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g) 
     for (int i = 0; i < T::FM; ++i)
 #pragma unroll
         for (int j = 0; j < T::FN; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-    float ra[T::FM][8], rb[T::B_IT][8];
+    ARegs ra;
+    float rb[T::B_IT][8];
     if (kbeg >= 0) {
-        load_a(kbeg, ra);
+        load_all_a(kbeg, ra);
         load_b(kbeg, rb);
     } else {
+        if constexpr (ASRC == A_SPLIT) load_all_a(kbeg, ra);
 #pragma unroll
-        for (int i = 0; i < T::FM; ++i)
+        for (int i = 0; i < (ASRC == A_SPLIT ? 0 : T::FM); ++i)
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const int k = kbeg + 8 * oct + j;
                 const size_t row = min(mw + 16 * i, g.M - 1);
-                ra[i][j] = k >= 0 ? (AT ? g.A[(size_t)k * g.lda + row] : g.A[row * g.lda + k]) : 0.f;
+                ra.f[i][j] = k >= 0 ? (AT ? g.A[(size_t)k * g.lda + row] : g.A[row * g.lda + k]) : 0.f;
             }
 #pragma unroll
         for (int i = 0; i < T::B_IT; ++i) bsrc.load_ragged(i, kbeg + 8 * b_oct[i], rb[i]);
@@ -299,7 +789,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g) 
     split_a(ra);
     store_b(bufs, rb);
     load_b(k_of(1), rb);
-    load_a(k_of(1), ra);
+    load_all_a(k_of(1), ra);
     __syncthreads();
     const int b_rd = oct * T::BN + wn * T::FN * 16 + r16;
     bf8 b[2][3];
@@ -313,10 +803,23 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g) 
     // part products, smallest first: (lo hi), (hi lo), (mid mid), (mid hi),
     // (hi mid), (hi hi)
     constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
-    constexpr int J_ST = T::FN > 8 ? 2 : 0; // column during which B's next stage is stored
+    // SPREAD: the conversions of the next stage, a pair of values at a time,
+    // over the columns, so that they run in the shadow of the MFMAs: B's pairs
+    // in the first half (before the barrier column), A's in the second, each
+    // item's next loads when its last pair is done (128 x 128 tiles: 128 x 4096
+    // x 4096 in 8 splits 42.5 -> 36.5 us, 1000 x 3001 x 2047 99 -> 80).  The
+    // 256 x 256 tile has no registers for A's converted next stage (9 spilled,
+    // 536 -> 564 us at 4096^3): B's are converted together during one column,
+    // A's after the last.
+    constexpr bool SPREAD = T::FM * T::FN <= 16;
+    constexpr int J_ST = SPREAD ? -1 : 2;
+    constexpr int NB = 4 * T::B_IT, NA = ASRC == A_SPLIT ? 0 : 4 * T::FM;
+    constexpr int B_COLS = NA ? T::FN / 2 : T::FN - 2, REST = T::FN - B_COLS;
+    u4 cb[3], an[T::FM][3];
     for (int s = 0; s < ns; ++s) {
         const u4 *Bc = bufs + (s & 1) * T::B_ST;
         u4 *Bn = bufs + ((s + 1) & 1) * T::B_ST;
+        const int k2 = k_of(s + 2);
 #pragma unroll
         for (int j = 0; j < T::FN; ++j) {
             // (the last column's reads for the next stage come after the
@@ -335,13 +838,37 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g) 
                 if (j > 0) acc[i][j - 1] += t[(j + 1) & 1][i];
             if (j == J_ST) {
                 store_b(Bn, rb);
-                load_b(k_of(s + 2), rb);
+                load_b(k2, rb);
+            }
+#pragma unroll
+            for (int u = 0; u < (SPREAD ? NB : 0); ++u) {
+                if (u * B_COLS / NB != j) continue;
+                split_pair(rb[u / 4], u % 4, cb, tiny);
+                if (u % 4 == 3) {
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) Bn[q * 4 * T::BN + b_slot[u / 4]] = cb[q];
+                    bsrc.load(u / 4, k2 + 8 * b_oct[u / 4], rb[u / 4]);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < (SPREAD ? NA : 0); ++u) {
+                if (B_COLS + u * REST / (NA ? NA : 1) != j) continue;
+                split_pair(ra.f[u / 4], u % 4, an[u / 4], tiny);
+                if (u % 4 == 3) load_a(k2, u / 4, ra);
             }
             if (j == T::FN - 2) __syncthreads();
-            // One operand read per FM MFMAs, then the adds of the column
-            // before (masks: 0x8 MFMA, 0x100 LDS read, 0x2 VALU): 4096^3 580
-            // -> 570 us against the compiler's order.
-            if (j != J_ST) {
+            // Operand reads between the first MFMAs, vector operations (the
+            // adds of the column before, conversions) after each of the
+            // others (masks: 0x8 MFMA, 0x100 LDS read, 0x2 VALU): 4096^3 580 ->
+            // 570 us against the compiler's order.
+            if constexpr (SPREAD) {
+#pragma unroll
+                for (int r = 0; r < 6 * T::FM; ++r) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    if (r % T::FM == T::FM - 1 && r < 3 * T::FM) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    if (r >= T::FM) __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                }
+            } else if (j != J_ST) {
 #pragma unroll
                 for (int r = 0; r < 3; ++r) {
                     __builtin_amdgcn_sched_group_barrier(0x008, T::FM, 0);
@@ -356,20 +883,28 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g) 
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        split_a(ra);
+        if constexpr (SPREAD && ASRC != A_SPLIT) {
+#pragma unroll
+            for (int i = 0; i < T::FM; ++i)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) a[i][q] = __builtin_bit_cast(bf8, an[i][q]);
+        } else {
+            split_a(ra);
+            load_all_a(k2, ra);
+        }
 #pragma unroll
         for (int i = 0; i < T::FM; ++i) acc[i][T::FN - 1] += t[(T::FN - 1) & 1][i];
-        load_a(k_of(s + 2), ra);
     }
 
-    bool bad = tiny.x < TINY || tiny.y < TINY;
+    bool bad = false;
 #pragma unroll
     for (int i = 0; i < T::FM; ++i)
 #pragma unroll
         for (int j = 0; j < T::FN; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
-    if (bad) *flag = 1;
+    if (bad) atomicOr(flag, (uint32_t)NOT_FINITE);
+    if (tiny.x < TINY || tiny.y < TINY) atomicOr(flag, (uint32_t)TINY_SEEN);
     __syncthreads();
     if constexpr (T::WK > 1) {
         f4 *red = reinterpret_cast<f4 *>(smem);
@@ -391,32 +926,19 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g) 
                     acc[i][j] += red[((q * T::GW + w) * T::FM * T::FN + i * T::FN + j) * 64 + lane];
     }
     const int nw = n0 + wn * T::FN * 16;
-    if (*flag) {
-        // In fp32: v_mfma_f32_16x16x4_f32, the same result layout.
-#pragma unroll
-        for (int i = 0; i < T::FM; ++i)
-#pragma unroll
-            for (int j = 0; j < T::FN; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-        for (int k0 = max(ks0, 0); k0 < kend; k0 += 4) {
-            const int k = k0 + oct;
-            float fa[T::FM], fb[T::FN];
-#pragma unroll
-            for (int i = 0; i < T::FM; ++i) {
+    if (*flag)
+        fp32_sums<T::FM, T::FN>(
+            acc, max(ks0, 0), kend, *flag & TINY_SEEN, oct,
+            [&](int i, int k) {
                 const size_t m = min(mw + 16 * i, g.M - 1);
-                fa[i] = k < kend ? (AT ? g.A[(size_t)k * g.lda + m] : g.A[m * g.lda + k]) : 0.f;
-            }
-#pragma unroll
-            for (int j = 0; j < T::FN; ++j)
-                fb[j] = k < kend ? BSrc::at(g, k, min(nw + 16 * j + r16, g.N - 1)) : 0.f;
-#pragma unroll
-            for (int i = 0; i < T::FM; ++i)
-#pragma unroll
-                for (int j = 0; j < T::FN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j], fa[i], acc[i][j], 0, 0, 0);
-        }
-    }
-    store_matrix<T::FM, T::FN>(g, acc, split, mw, nw + 4 * oct);
+                if constexpr (ASRC == A_SPLIT) return conv_weight(g, cv, (int)m, k);
+                return AT ? g.A[(size_t)k * g.lda + m] : g.A[m * g.lda + k];
+            },
+            [&](int j, int k) { return BSrc::at(g, cv, k, min(nw + 16 * j + r16, g.N - 1)); });
+    if constexpr (OUT == OUT_MATRIX)
+        store_matrix<T::FM, T::FN>(g, acc, split, mw, nw + 4 * oct);
+    else
+        store_conv<T::FM, T::FN, OUT == OUT_POOL>(g, cv, acc, split, mw, nw + 4 * oct);
 }
 
 // C = sum of the K splits' partials [split][M][N] in split order, then bias
@@ -450,10 +972,48 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(SplitGemm g, int spli
     }
 }
 
+// The splits' partials of a convolution, in split order, then its epilogue; a
+// thread per 4 columns of a channel.
+template <bool POOL>
+__global__ __launch_bounds__(256) void split_conv_reduce_kernel(SplitGemm g, SplitConv c, int splits) {
+    const int quads = (g.N + 3) / 4;
+    const size_t total = (size_t)g.M * g.N;
+    for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < (size_t)g.M * quads;
+         q += (size_t)gridDim.x * blockDim.x) {
+        const int row = (int)(q / quads), n = 4 * (int)(q - (size_t)row * quads);
+        const float *src = g.partial + (size_t)row * g.N + n;
+        const bool whole = n + 3 < g.N;
+        f4 s = {0.f, 0.f, 0.f, 0.f};
+        for (int z0 = 0; z0 < splits; z0 += 8) {
+            f4 t[8]; // up to 8 loads in flight
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (z0 + u >= splits) continue;
+                const float *p = src + (z0 + u) * total;
+                if (whole)
+                    t[u] = *reinterpret_cast<const f4u *>(p);
+                else
+                    for (int v = 0; v < 4; ++v) t[u][v] = n + v < g.N ? p[v] : 0.f;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (z0 + u < splits) s = z0 + u ? s + t[u] : t[u];
+        }
+        store_conv_quad<POOL>(g, c, s, row, n, ConvColumn(n, POOL ? 4 * c.PP : c.P),
+                              (g.flags & CAMEL_EPI_BIAS) ? g.bias[row] : 0.f);
+    }
+}
+
 // 256 x 256: 8 waves of 32 x 256.  128 x 128: 8 waves, 4 of 32 x 128 on each of
 // two k groups.
 using T256 = STile<2, 16, 8, 1, 1>;
 using T128 = STile<2, 8, 4, 1, 2>;
+
+// Convolutions: 4 waves of 32 channels x 128 pixels (two work-groups share a
+// CU, so one's first loads and stores overlap the other's products), 2 x 2 of
+// 32 x 64 for up to 64 channels.
+using C128 = STile<2, 8, 4, 1, 1>;
+using C64 = STile<2, 4, 2, 2, 1>;
 
 // K per split and the splits a request really gives: whole steps, none empty.
 template <class T> void split_k(int64_t K, int splits, int &k_per_split, int &used) {
@@ -470,9 +1030,11 @@ template <class T> int launch(SplitGemm g, bool a_trans, int splits) {
     if (used == 1) g.partial = nullptr;
     const dim3 grid(tiles, (unsigned)used), block(T::THREADS);
     if (a_trans)
-        hipLaunchKernelGGL((split_gemm_kernel<T, true>), grid, block, 0, stream(), g);
+        hipLaunchKernelGGL((split_gemm_kernel<T, A_COLS, MatrixB<T>, OUT_MATRIX>), grid, block, 0, stream(), g,
+                           SplitConv{});
     else
-        hipLaunchKernelGGL((split_gemm_kernel<T, false>), grid, block, 0, stream(), g);
+        hipLaunchKernelGGL((split_gemm_kernel<T, A_ROWS, MatrixB<T>, OUT_MATRIX>), grid, block, 0, stream(), g,
+                           SplitConv{});
     CAMEL_RETURN_IF(check_launch("split_gemm_kernel"));
     if (used > 1) {
         const bool vec = g.N % 4 == 0 && ((uintptr_t)g.C & 15) == 0;
@@ -482,6 +1044,98 @@ template <class T> int launch(SplitGemm g, bool a_trans, int splits) {
         else
             hipLaunchKernelGGL(split_reduce_kernel<false>, dim3(grid_for(items, 256)), dim3(256), 0, stream(), g, used);
         CAMEL_RETURN_IF(check_launch("split_reduce_kernel"));
+    }
+    return CAMEL_HIP_OK;
+}
+
+template <class T> int64_t conv_tiles(const SplitGemm &g) {
+    return ((int64_t)(g.M + T::BM - 1) / T::BM) * ((g.N + T::BN - 1) / T::BN);
+}
+
+// K splits of a convolution: few tiles with many stages (small batches) leave
+// the chip idle.  Estimates from measured calls, in us: a stage takes 1.9 alone
+// on its CU and 3.2 beside a second work-group, a work-group 6 besides, the
+// partials 3 and their traffic.  (1 x 128 x 14 x 14 -> 256 3x3, 4 tiles of 36
+// stages: unsplit 80.)
+int conv_splits(const SplitGemm &g, int64_t tiles, int cus) {
+    const int stages = (g.K + BK - 1) / BK;
+    int best = 1;
+    double best_t = 1e30;
+    for (int want = 1; want <= 16; ++want) {
+        const int per = (stages + want - 1) / want, used = (stages + per - 1) / per;
+        const size_t bytes = used > 1 ? (size_t)used * g.M * g.N * sizeof(float) : 0;
+        if (used != want || (want > 1 && per < 3) || bytes > CAMEL_HIP_NOALLOC_SCRATCH_BYTES) continue;
+        const int64_t wgs = tiles * used;
+        const double t = (wgs <= cus ? 6 + 1.9 * per : (double)((wgs + 2 * cus - 1) / (2 * cus)) * (6 + 3.2 * per)) +
+                         (used > 1 ? 3 + 2.0 * bytes / 6e6 : 0);
+        if (t < best_t) {
+            best_t = t;
+            best = used;
+        }
+    }
+    return best;
+}
+
+template <class T, bool QUADS> int launch_patch(const SplitGemm &g, const SplitConv &c, bool pool) {
+    const int64_t per = pool ? 4 * c.PP : c.P;
+    const int64_t tiles_n =
+        c.per_image ? g.N / per * ((per + T::BN - 1) / T::BN) : ((int64_t)g.N + T::BN - 1) / T::BN;
+    const dim3 grid((unsigned)((g.M + T::BM - 1) / T::BM * tiles_n)), block(T::THREADS);
+    if (pool)
+        hipLaunchKernelGGL((conv_patch_kernel<T, QUADS, true>), grid, block, 0, stream(), g, c);
+    else
+        hipLaunchKernelGGL((conv_patch_kernel<T, QUADS, false>), grid, block, 0, stream(), g, c);
+    return check_launch("conv_patch_kernel");
+}
+
+// K in runs of 32 channels, which the patch kernel needs: stride 1, several taps,
+// channels that fill blocks of 32 (at most 1/8 padding) and 128-pixel tiles for
+// 3/4 of the CUs without K splits.  Decided on the geometry alone, so
+// that all layouts and the pooled form sum in the same order.
+bool conv_blocked(const SplitConv &c, int64_t pixels, int64_t Co, int cus) {
+    const int64_t blocks = (c.C + BK - 1) / BK, tile_m = Co <= 64 ? 64 : 128;
+    return c.stride == 1 && c.KH * c.KW >= 4 && blocks * BK * 8 <= (int64_t)c.C * 9 &&
+           (pixels + 127) / 128 * ((Co + tile_m - 1) / tile_m) * 4 >= 3 * cus;
+}
+
+// Positions a patch needs for any tile of 128 columns, 0 if over PATCH:
+// `wraps` row ends (pool order: ends of two-row strips of windows) each add
+// the padding between rows, the taps reach further down, and a tile across
+// images adds the rows between them -- or tiles stay within images, where that
+// wastes at most 1/8 of their columns.
+int patch_positions(const SplitConv &c, int64_t images, bool pool, int &per_image) {
+    constexpr int64_t BN = 128;
+    const int64_t Wp = c.W + 2 * c.pad, OW = c.OW, PW = c.PW, per = pool ? 4 * c.PP : c.P;
+    if ((images * (int64_t)(c.H + 2 * c.pad) + 1) * Wp + PATCH >= INT32_MAX) return 0;
+    const int64_t reach = (c.KH - 1) * Wp + c.KW;
+    const int64_t inside =
+        reach + (pool ? (2 * ((BN / 4 + PW - 2) / PW) + 1) * Wp + OW : BN + (BN + OW - 2) / OW * (Wp - OW));
+    const int64_t across = inside + (BN + per - 2) / per * c.KH * Wp;
+    per_image = across > PATCH;
+    if (!per_image) return (int)across;
+    return inside <= PATCH && (per + BN - 1) / BN * BN * 8 <= per * 9 ? (int)inside : 0;
+}
+
+template <class T, bool QUADS>
+int launch_conv(SplitGemm g, const SplitConv &c, bool pool, int splits, float *partial) {
+    int used = 1;
+    split_k<T>(g.K, splits, g.k_per_split, used);
+    g.partial = used > 1 ? partial : nullptr;
+    const dim3 grid((unsigned)conv_tiles<T>(g), (unsigned)used), block(T::THREADS);
+    if (pool)
+        hipLaunchKernelGGL((split_gemm_kernel<T, A_SPLIT, ConvB<T, QUADS, true>, OUT_POOL>), grid, block, 0,
+                           stream(), g, c);
+    else
+        hipLaunchKernelGGL((split_gemm_kernel<T, A_SPLIT, ConvB<T, QUADS, false>, OUT_CONV>), grid, block, 0,
+                           stream(), g, c);
+    CAMEL_RETURN_IF(check_launch("split_gemm_kernel (conv)"));
+    if (used > 1) {
+        const dim3 rgrid(grid_for((int64_t)g.M * ((g.N + 3) / 4), 256));
+        if (pool)
+            hipLaunchKernelGGL(split_conv_reduce_kernel<true>, rgrid, dim3(256), 0, stream(), g, c, used);
+        else
+            hipLaunchKernelGGL(split_conv_reduce_kernel<false>, rgrid, dim3(256), 0, stream(), g, c, used);
+        CAMEL_RETURN_IF(check_launch("split_conv_reduce_kernel"));
     }
     return CAMEL_HIP_OK;
 }
@@ -524,7 +1178,7 @@ SplitPlan split_gemm_plan(int64_t M, int64_t N, int64_t K, bool unaligned, int64
         }
     };
     consider(SplitTile::T256, 256, T256::SB, 8.5, 4.1);
-    consider(SplitTile::T128, 128, T128::SB, 7.0, 2.8);
+    consider(SplitTile::T128, 128, T128::SB, 7.0, 2.4);
     return best;
 }
 
@@ -532,6 +1186,66 @@ int split_gemm(SplitGemm g, bool a_trans, const SplitPlan &plan, float *partial)
     g.partial = partial;
     if (plan.tile == SplitTile::T256) return launch<T256>(g, a_trans, plan.splits);
     return launch<T128>(g, a_trans, plan.splits);
+}
+
+bool split_conv_serves(int64_t N, int64_t C, int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW,
+                       int64_t pad) {
+    const int64_t C8 = (C + 7) / 8 * 8, K = C8 * KH * KW;
+    // 32 taps in a lane's mask; the divisions by C8 and KW and the buffer's
+    // offsets (x, the reach of the first window, padded channels) stay exact;
+    // channels padded by at most 1.6
+    return C >= 5 && KH * KW <= 32 && K >= 64 && K < 65536 && Co >= 16 &&
+           (N * C8 * H * W + 2 * pad * (W + 1) * C8) * 4 < (int64_t)1 << 30;
+}
+
+SplitConvPlan split_conv_plan(const SplitGemm &g, const SplitConv &c, bool pool, int cus) {
+    SplitConvPlan p;
+    if (conv_blocked(c, g.N, g.M, cus)) {
+        p.blocked = 1;
+        p.patch = patch_positions(c, g.N / c.P, pool, p.per_image);
+        p.weight_bytes = (size_t)((c.C + BK - 1) / BK) * c.KH * c.KW * ((g.M + 15) / 16) * 3072;
+        return p;
+    }
+    p.splits = conv_splits(g, g.M <= 64 ? conv_tiles<C64>(g) : conv_tiles<C128>(g), cus);
+    p.weight_bytes = (size_t)((g.K + BK - 1) / BK) * ((g.M + 15) / 16) * 3072;
+    p.partial_bytes = p.splits > 1 ? (size_t)p.splits * g.M * g.N * sizeof(float) : 0;
+    return p;
+}
+
+int split_conv(SplitGemm g, SplitConv c, bool quads, bool pool, const SplitConvPlan &plan, void *scratch) {
+    if (pool) g.N = g.N / c.P * c.PP * 4;
+    c.shift = c.pad * (c.W + 1) * c.pxs;
+    c.patch = plan.patch;
+    c.per_image = plan.per_image;
+    c.taps = c.KH * c.KW;
+    c.unit = plan.blocked ? BK : (c.C + 7) / 8 * 8;
+    auto mul = [](int d) { return (uint32_t)(((uint64_t)1 << 32) / d + 1); };
+    c.mul_unit = mul(c.unit);
+    c.mul_kw = mul(c.KW);
+    c.mul_taps = mul(c.taps);
+    if (plan.blocked) g.K = (c.C + BK - 1) / BK * c.taps * BK;
+    const int stages = (g.K + BK - 1) / BK;
+    c.kpad = stages * BK - g.K;
+    c.w_split = static_cast<const u4 *>(scratch);
+    float *partial = reinterpret_cast<float *>(static_cast<char *>(scratch) + plan.weight_bytes);
+    hipLaunchKernelGGL(split_weights_kernel, dim3(stages, (g.M + 15) / 16), dim3(64), 0, stream(), g, c,
+                       static_cast<u4 *>(scratch));
+    CAMEL_RETURN_IF(check_launch("split_weights_kernel"));
+    if (plan.patch) {
+        g.partial = nullptr;
+        c.shift = 0;
+        c.bytes = (uint32_t)((int64_t)(pool ? g.N / (4 * c.PP) : g.N / c.P) * c.CHW * 4);
+        if (g.M <= 64)
+            return quads ? launch_patch<PatchTile<2, 4, 2, 2>, true>(g, c, pool)
+                         : launch_patch<PatchTile<2, 4, 2, 2>, false>(g, c, pool);
+        return quads ? launch_patch<PatchTile<2, 8, 4, 1>, true>(g, c, pool)
+                     : launch_patch<PatchTile<2, 8, 4, 1>, false>(g, c, pool);
+    }
+    if (g.M <= 64)
+        return quads ? launch_conv<C64, true>(g, c, pool, plan.splits, partial)
+                     : launch_conv<C64, false>(g, c, pool, plan.splits, partial);
+    return quads ? launch_conv<C128, true>(g, c, pool, plan.splits, partial)
+                 : launch_conv<C128, false>(g, c, pool, plan.splits, partial);
 }
 
 } // namespace camel_hip

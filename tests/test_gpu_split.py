@@ -123,3 +123,92 @@ def test_special_values_propagate(M, N, Kd, trans):
     assert np.array_equal(np.isnan(got), np.isnan(ref))
     assert np.array_equal(np.isposinf(got), np.isposinf(ref))
     assert np.array_equal(np.isneginf(got), np.isneginf(ref))
+
+
+# ---- convolutions ------------------------------------------------------------
+
+# N, C, H, W, Co, KH, KW, stride, pad: which kernel and what is ragged
+CONVS = [
+    (8, 32, 56, 56, 64, 3, 3, 1, 1),     # patch kernel, tiles within images (the last of 64 pixels)
+    (16, 64, 28, 28, 200, 3, 3, 1, 1),   # patch, tiles across images, Co % 128 = 72
+    (45, 31, 17, 19, 130, 3, 2, 1, 2),   # patch, 31 of 32 channels, odd everything
+    (8, 32, 120, 120, 20, 5, 5, 1, 0),   # 32-channel runs, patch too long: im2col loads
+    (5, 13, 33, 31, 47, 5, 5, 2, 2),     # im2col loads, channels padded to 16, K splits
+    (2, 100, 9, 7, 130, 1, 1, 1, 0),     # one tap, K % 32 = 8: stage below k = 0
+    (1, 256, 7, 7, 96, 3, 3, 1, 1),      # many K splits of one tile of 49 pixels
+]
+
+
+def conv(x, w, bias, geom, flags, pool=False, layout=0):
+    N, C, H_, W_, Co, KH, KW, st, pad = geom
+    OH, OW = (H_ + 2 * pad - KH) // st + 1, (W_ + 2 * pad - KW) // st + 1
+    shape = (N, Co, OH // 2, OW // 2) if pool else (N, Co, OH, OW)
+    if layout == H.CONV_X_NCHW4:
+        x = x.reshape(N, C // 4, 4, H_, W_).transpose(0, 1, 3, 4, 2)
+    elif layout == H.CONV_X_NHWC:
+        x = x.transpose(0, 2, 3, 1)
+    dx, dw = K.dev(x), K.dev(w)
+    db = K.dev(bias) if bias is not None else None
+    dy = K.empty(int(np.prod(shape)) * 4)
+    H.call("camel_hip_conv2d_pool2" if pool else "camel_hip_conv2d", K.P(dx.ptr), K.P(dw.ptr),
+           K.P(db.ptr) if db is not None else None, K.P(dy.ptr), *geom, flags | layout)
+    return K.host(dy, F, shape)
+
+
+def pooled(y):
+    n, c, h, w = y.shape
+    y = y[:, :, :h // 2 * 2, :w // 2 * 2].reshape(n, c, h // 2, 2, w // 2, 2)
+    out = y[:, :, :, 0, :, 0]
+    for dy, dx in ((0, 1), (1, 0), (1, 1)):
+        out = np.where(y[:, :, :, dy, :, dx] > out, y[:, :, :, dy, :, dx], out)
+    return out
+
+
+@pytest.mark.parametrize("geom", CONVS)
+def test_conv_exact_on_wide_operands(geom):
+    from tests.test_gpu_exact import exact_conv, ternary
+    N, C, H_, W_, Co, KH, KW, st, pad = geom
+    print(f"split conv {geom}", flush=True)
+    for side in ("x", "w"):
+        if side == "x":
+            x = wide(0x5200 + C, (N, C, H_, W_), -1023, 1023)
+            w = ternary(0x5201 + Co, (Co, C * KH * KW), 1).reshape(Co, C, KH, KW)
+        else:
+            x = ternary(0x5202 + C, (N, C, H_, W_), 1)
+            w = wide(0x5203 + Co, (Co, C, KH, KW), -1023, 1023)
+        bias = wide(0x5204, (Co,))
+        want = exact_conv(x, w, bias, st, pad, True)
+        assert_bits(conv(x, w, bias, geom, EPI), want, f"wide {side}")
+        if want.shape[2] >= 2 and want.shape[3] >= 2:
+            assert_bits(conv(x, w, bias, geom, EPI, pool=True), pooled(want), f"wide {side}, pooled")
+
+
+@pytest.mark.parametrize("geom", CONVS)
+def test_conv_layouts_pool_and_special_values(geom):
+    # Random floats with a few special and out-of-range values: the layouts and
+    # the pooled form agree bit for bit (non-finite sums are formed again one
+    # by one, whatever the tile), and non-finite outputs sit where the fp64
+    # convolution has them.
+    N, C, H_, W_, Co, KH, KW, st, pad = geom
+    print(f"split conv special {geom}", flush=True)
+    rng = np.random.default_rng(C + Co)
+    x = rng.uniform(-1, 1, (N, C, H_, W_)).astype(F)
+    w = rng.uniform(-1, 1, (Co, C, KH, KW)).astype(F)
+    bias = rng.uniform(-1, 1, Co).astype(F)
+    x[0, 0, 0, 0], x[-1, -1, -1, -1], x[0, C // 2, H_ // 2, W_ // 2] = np.inf, np.nan, -np.inf
+    y = conv(x, w, bias, geom, H.EPI_BIAS)
+    if C % 4 == 0:
+        for layout in (H.CONV_X_NHWC, H.CONV_X_NCHW4):
+            np.testing.assert_array_equal(conv(x, w, bias, geom, H.EPI_BIAS, layout=layout), y)
+    if min(y.shape[2:]) >= 2:
+        np.testing.assert_array_equal(conv(x, w, bias, geom, H.EPI_BIAS, pool=True), pooled(y))
+    # the non-finite outputs: the windows that hold a special value
+    xf = np.where(np.isfinite(x), 0, 1).astype(F)
+    touched = conv(xf, np.ones_like(w), None, geom, 0) > 0
+    assert np.array_equal(~np.isfinite(y), touched)
+    # values below the split's range: fp32 to the fp32 kernels' bound
+    x = np.where(np.isfinite(x), x, 0).astype(F)
+    base = conv(x, w, None, geom, 0)
+    tiny = conv(x * F(2.0 ** -112), w, None, geom, 0).astype(np.float64) * 2.0 ** 112
+    bound = 1e-5 * np.sqrt(C * KH * KW) * conv(np.abs(x), np.abs(w), None, geom, 0)
+    assert np.all(np.abs(tiny - base) <= bound)
