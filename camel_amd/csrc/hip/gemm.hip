@@ -2610,236 +2610,6 @@ void choose(int64_t M, int64_t N, int64_t K, int cus, Cfg &cfg, int &splits, int
     }
 }
 
-// ---- the first two convolutions of an image CNN, fused with the pool -----------
-//
-// y = maxpool2x2(conv2(conv1(x))) (each conv with its optional bias and relu)
-// for a one-channel input: conv1 1 -> CP_C1 channels, 3x3, then conv2
-// CP_C1 -> Co2, 3x3, both stride 1 and unpadded, then the 2x2 stride-2 pool.
-// conv1's output (CP_C1 x 26 x 26 per 28 x 28 image, 44 MB at batch 512)
-// never reaches HBM: a work-group computes the rows of it that its band of
-// conv2 rows reads into LDS, then runs conv2 as an implicit GEMM whose B
-// operand is read straight from that LDS patch, and stores only the pooled
-// values.
-//   * work-group = (image, band of CP_BR pooled rows = 2 CP_BR conv2 rows) x
-//     64 output channels; 4 waves as 2 (channels) x 2 (column halves), each
-//     wave 32 channels x CP_NBW blocks of 32 columns;
-//   * columns in pool order, 4 per window ((0,0), (0,1), (1,0), (1,1)), so a
-//     window is one DPP quad and the epilogue takes its max in registers,
-//     and 16 consecutive columns a 2 x 2 block of windows (cp_window);
-//   * conv1 is the direct kernel's FMA chain (k = (kh, kw) ascending, then
-//     bias and x * (x > 0)), so the patch holds exactly the values the conv1
-//     kernel stores;
-//   * conv2's A operand (weights packed [Co2][3][3][CP_C1]) is held in
-//     registers for all of K; the MFMA sequence -- K in (kh, kw, c) order,
-//     8-channel groups, each 32x32x2 MFMA pairing channels c and c + 4 --
-//     and the epilogue (bias, relu, strict-'>' window max) are those of the
-//     implicit GEMM with the pooled NCHW4 loader, so the result equals the
-//     two conv calls and the pool bit for bit.
-constexpr int CP_C1 = 32;                 // conv1 output channels = conv2 input channels
-constexpr int CP_W = 28;                  // input width
-constexpr int CP_OW1 = CP_W - 2;          // conv1 output width (26)
-constexpr int CP_PW = (CP_OW1 - 2) / 2;   // pooled width (12)
-constexpr int CP_BR = 4;                  // pooled rows per work-group
-constexpr int CP_R1 = 2 * CP_BR + 2;      // conv1 rows a band reads (10)
-constexpr int CP_IR = CP_R1 + 2;          // input rows a band reads (12)
-// The patch is stored by channel quads, [C1/4][CP_R1][CP_RS][4]: a lane reads
-// the 4 channels of one pixel that 4 consecutive MFMAs take with one 16-byte
-// read.  A 16-byte LDS read serves 16 lanes per clock, conflict-free when
-// their chunks are distinct mod 16 (64 banks x 4 bytes); those 16 lanes read
-// a 2 x 2 block of windows, pixels (2 py + r, 2 px + c) for r, c in 0..3, and
-// with a row pitch of CP_RS = 28 pixels (28 r = 0, 12, 8, 4 mod 16) the 16
-// chunks are distinct.  (4 windows of one row, 2 rows x 8 pixels, put 4
-// chunks on 2 lanes each at this pitch; a pitch of 40 separates those too but
-// ran the CNN forward 1.7% slower; the 2 x 2 blocks ran it 0.4% faster.  The
-// kernel's SQ_LDS_BANK_CONFLICT share reads 28.5% with either mapping at this
-// pitch and 0 at pitch 40, so what that counter counts here is not explained
-// by this model of the patch reads.)
-constexpr int CP_RS = 28;
-static_assert(CP_RS >= CP_OW1 && CP_RS % 16 == 12, "conflict-free patch row pitch");
-// One channel quad of the patch: 1120 floats, padded to 1124 (= 4 mod 32) so
-// that the conv1 phase's 32 lanes, one channel each, store one pixel to 32
-// distinct banks.
-constexpr int CP_QPLANE = CP_R1 * CP_RS * 4 + 4;
-constexpr int CP_COLS = CP_BR * CP_PW * 4; // GEMM columns of a band (192)
-constexpr int CP_NBW = CP_COLS / 32 / 2;  // 32-column blocks per wave (3)
-static_assert(CP_COLS % 64 == 0, "a band is whole 32-column blocks for both column halves");
-
-// The pool window (row py of the band, column px) of GEMM column col: 4
-// columns per window, and 16 consecutive columns a 2 x 2 block of windows.
-__device__ __forceinline__ void cp_window(int col, int &py, int &px) {
-    static_assert(CP_BR % 2 == 0 && CP_PW % 2 == 0, "windows in 2 x 2 blocks");
-    const int g = col >> 4, w4 = (col >> 2) & 3;
-    py = 2 * (g / (CP_PW / 2)) + (w4 >> 1);
-    px = 2 * (g % (CP_PW / 2)) + (w4 & 1);
-}
-
-__global__ __launch_bounds__(256, 2) void conv_pair_pool_kernel(
-    const float *__restrict__ x, const float *__restrict__ w1, const float *__restrict__ b1,
-    const float *__restrict__ w2p, const float *__restrict__ b2, float *__restrict__ y, int H,
-    int Co2, int bands, int flags1, int flags2) {
-    const bool BIAS1 = flags1 & CAMEL_EPI_BIAS, RELU1 = flags1 & CAMEL_EPI_RELU;
-    const bool BIAS2 = flags2 & CAMEL_EPI_BIAS, RELU2 = flags2 & CAMEL_EPI_RELU;
-    __shared__ __attribute__((aligned(16))) float patch[CP_C1 / 4 * CP_QPLANE];
-    __shared__ __attribute__((aligned(16))) float img[CP_IR * CP_W];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int half = lane >> 5, r32 = lane & 31;
-    const int wm = wave & 1, wn = wave >> 1;
-    const int n = blockIdx.x / bands, band = blockIdx.x - n * bands;
-    const int m0 = blockIdx.y * 64;
-    const int PH = bands * CP_BR;
-    const int Y0 = band * 2 * CP_BR; // first conv2 (and conv1) row of the band
-
-    // conv2 weights of this lane's row as the MFMA A operand, one (kh, kw)
-    // at a time: a[buf][s8] holds channels 8 s8 + 4 half .. +3 (from L2,
-    // two (kh, kw) ahead of their use).
-    const float *wr = w2p + (size_t)(m0 + 32 * wm + r32) * 9 * CP_C1 + 4 * half;
-    float4 a[3][CP_C1 / 8];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int s8 = 0; s8 < CP_C1 / 8; ++s8)
-            a[j][s8] = *reinterpret_cast<const float4 *>(wr + j * CP_C1 + 8 * s8);
-
-    // conv1's weights and bias for this lane's channel (lane r32 computes
-    // channel r32 of one pixel; the two half-waves take two pixels).
-    float w1r[9];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) w1r[k] = w1[r32 * 9 + k];
-    const float b1r = BIAS1 ? b1[r32] : 0.f;
-
-    // The input rows of the band, 16 bytes per thread (zeros past the image:
-    // never read by a valid output, since the bands tile the pooled rows).
-    {
-        const float4 *xi = reinterpret_cast<const float4 *>(x + ((size_t)n * H + Y0) * CP_W);
-        if (tid < CP_IR * CP_W / 4) {
-            const int r = Y0 + tid / (CP_W / 4);
-            reinterpret_cast<float4 *>(img)[tid] = r < H ? xi[tid] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    }
-    __syncthreads();
-
-    // conv1 into the patch: the direct kernel's FMA chain, then bias and relu.
-    for (int p = 2 * wave + half; p < CP_R1 * CP_OW1; p += 8) {
-        const int r = p / CP_OW1, c = p - r * CP_OW1;
-        float acc = 0.f;
-#pragma unroll
-        for (int kh = 0; kh < 3; ++kh)
-#pragma unroll
-            for (int kw = 0; kw < 3; ++kw)
-                acc = __builtin_fmaf(w1r[kh * 3 + kw], img[(r + kh) * CP_W + c + kw], acc);
-        if (BIAS1) acc = acc + b1r;
-        if (RELU1) acc = relu_idiom(acc);
-        patch[(r32 >> 2) * CP_QPLANE + (r * CP_RS + c) * 4 + (r32 & 3)] = acc;
-    }
-    __syncthreads();
-
-    // conv2: lane (r32, half) reads B[k][col] for channels 8 s8 + 4 half + t,
-    // t = 0..3, of pixel (oy + kh, ox + kw) of its column col of each block:
-    // one 16-byte read of channel quad 2 s8 + half.
-    int base[CP_NBW];
-#pragma unroll
-    for (int b = 0; b < CP_NBW; ++b) {
-        const int col = 32 * (CP_NBW * wn + b) + r32, d = col & 3;
-        int py, px;
-        cp_window(col, py, px);
-        base[b] = half * CP_QPLANE + ((2 * py + (d >> 1)) * CP_RS + 2 * px + (d & 1)) * 4;
-    }
-    floatx16 acc[CP_NBW];
-#pragma unroll
-    for (int b = 0; b < CP_NBW; ++b)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[b][v] = 0.f;
-    // Each 8-channel group of a (kh, kw) stage loads the same group's weights
-    // of stage + 2 and reads the next group's patch values, spread over its
-    // own MFMAs: one patch read per two MFMAs, then the weight load
-    // (scheduling group barriers keep that order; 4% faster over the CNN
-    // forward than the reads together ahead of the MFMAs and the stage's
-    // weight loads together at its start).
-    auto patch_reads = [&](int khw, int s8, float4 *bv) {
-        const int kh = khw / 3, kw = khw - 3 * (khw / 3);
-        const int off = 2 * s8 * CP_QPLANE + (kh * CP_RS + kw) * 4;
-#pragma unroll
-        for (int b = 0; b < CP_NBW; ++b)
-            bv[b] = *reinterpret_cast<const float4 *>(patch + base[b] + off);
-    };
-    float4 bv[2][CP_NBW];
-    patch_reads(0, 0, bv[0]);
-#pragma unroll
-    for (int khw = 0; khw < 9; ++khw) {
-        const int cur = khw % 3;
-#pragma unroll
-        for (int s8 = 0; s8 < CP_C1 / 8; ++s8) {
-            const int g = khw * (CP_C1 / 8) + s8; // group index over all of K
-            const bool next = g + 1 < 9 * (CP_C1 / 8);
-            const bool ahead = khw + 2 < 9;
-            // group s8's weights of stage khw + 2
-            if (ahead)
-                a[(khw + 2) % 3][s8] =
-                    *reinterpret_cast<const float4 *>(wr + (khw + 2) * CP_C1 + 8 * s8);
-            if (next) patch_reads((g + 1) / (CP_C1 / 8), (g + 1) % (CP_C1 / 8), bv[(g + 1) & 1]);
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int b = 0; b < CP_NBW; ++b)
-                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[cur][s8][t], bv[g & 1][b][t],
-                                                                  acc[b], 0, 0, 0);
-            if (next) {
-                // one patch read per two MFMAs at the head of the group, then
-                // the weight load after one more MFMA (masks: 0x100 LDS read,
-                // 0x20 global read, 0x8 MFMA)
-#pragma unroll
-                for (int r = 0; r < CP_NBW; ++r) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                }
-                if (ahead) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, 2 * CP_NBW - 1, 0);
-                } else {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 2 * CP_NBW, 0);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-
-    // Epilogue: bias, relu, then the window max over the lane quad in the
-    // order (0,0), (0,1), (1,0), (1,1) with a strict '>'; the quad's first
-    // lane stores the pooled value.
-    float brow[16];
-#pragma unroll
-    for (int v = 0; v < 16; ++v)
-        brow[v] = BIAS2 ? b2[m0 + 32 * wm + 8 * (v >> 2) + 4 * half + (v & 3)] : 0.f;
-#pragma unroll
-    for (int b = 0; b < CP_NBW; ++b) {
-        const int col = 32 * (CP_NBW * wn + b) + r32;
-        int py, px;
-        cp_window(col, py, px);
-        py += band * CP_BR;
-        float *out = y + ((size_t)n * Co2 + m0 + 32 * wm) * PH * CP_PW + (size_t)py * CP_PW + px;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int row = 8 * (v >> 2) + 4 * half + (v & 3);
-            float xo = acc[b][v];
-            if (BIAS2) xo = xo + brow[v];
-            if (RELU2) xo = relu_idiom(xo);
-            const float x1 = quad_lane<1>(xo), x2 = quad_lane<2>(xo), x3 = quad_lane<3>(xo);
-            float mx = xo;
-            if (x1 > mx) mx = x1;
-            if (x2 > mx) mx = x2;
-            if (x3 > mx) mx = x3;
-            if ((r32 & 3) == 0) out[(size_t)row * PH * CP_PW] = mx;
-        }
-    }
-}
-
-// True when conv_pair_pool_kernel serves the pair.
-bool conv_pair_supported(int64_t H, int64_t W, int64_t C1, int64_t Co2) {
-    return W == CP_W && C1 == CP_C1 && Co2 > 0 && Co2 % 64 == 0 && H >= 6 &&
-           (H - 4) % (2 * CP_BR) == 0;
-}
-
 // ---- conv2d host paths -----------------------------------------------------------
 
 // Activation layouts of the conv paths: NCHW (the tensor layout), NHWC and
@@ -3081,14 +2851,6 @@ int conv2d_gather(const float *x, const float *w, const float *bias, float *y, i
     return ok();
 }
 
-// True when conv2d runs on the split-operand kernels.  The first layers of an
-// image CNN that conv_pair_pool_kernel serves keep its fp32 MFMA sequence.
-bool conv_on_split(int64_t N, int64_t C, int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW,
-                   int64_t stride, int64_t pad) {
-    const bool pair_layer = C == CP_C1 && KH == 3 && KW == 3 && stride == 1 && pad == 0 && Co % 64 == 0;
-    return !pair_layer && split_conv_serves(N, C, H, W, Co, KH, KW, pad);
-}
-
 // conv2d on the split-operand kernels: x in any layout (NHWC and NCHW4 with
 // C % 4 == 0 and 16-byte alignment), y NCHW, NCHW4 (flags) or pooled.
 int conv2d_split(const float *x, const float *w, const float *bias, float *y, int64_t N, int64_t C,
@@ -3199,7 +2961,7 @@ int conv2d_run(const float *x, const float *w, const float *bias, float *y, int6
         flags &= ~CAMEL_CONV_W_PACKED;
     }
     // out_flags: the epilogue flags, plus CAMEL_CONV_Y_NCHW4 for an NCHW4 out
-    const bool split = conv_on_split(N, C, H, W, Co, KH, KW, stride, pad);
+    const bool split = split_conv_serves(N, C, H, W, Co, KH, KW, pad);
     auto nhwc_gemm = [&](float *out, bool pooled, int out_flags) -> int {
         if (split)
             return conv2d_split(x, w, bias, out, N, C, H, W, Co, KH, KW, stride, pad, OH, OW, out_flags, xl,
@@ -3622,7 +3384,7 @@ int camel_hip_conv2d_pair_pool2(const float *x, const float *w1, const float *b1
     if ((flags1 & ~(CAMEL_EPI_BIAS | CAMEL_EPI_RELU)) ||
         (flags2 & ~(CAMEL_EPI_BIAS | CAMEL_EPI_RELU | CAMEL_CONV_W_PACKED)))
         return fail(CAMEL_HIP_ERR_ARG, std::string(who) + ": unknown flags");
-    if (!conv_pair_supported(H, W, C1, Co2) || N > INT32_MAX / 64 ||
+    if (!split_pair_serves(H, W, C1, Co2) || N > INT32_MAX / 64 ||
         !product_fits({N, Co2, (H - 4) / 2, (W - 4) / 2}))
         return fail(CAMEL_HIP_ERR_SHAPE,
                     std::string(who) + ": shape not served (needs W = 28, C1 = 32, Co2 % 64 == 0, "
@@ -3635,20 +3397,21 @@ int camel_hip_conv2d_pair_pool2(const float *x, const float *w1, const float *b1
         return fail(CAMEL_HIP_ERR_ARG, std::string(who) + ": x and w2 must be 16-byte aligned");
     CAMEL_LOCK();
     CAMEL_INIT_OR_RETURN();
-    const float *w2p = w2;
-    Scratch packed;
-    if (!(flags2 & CAMEL_CONV_W_PACKED)) {
-        CAMEL_RETURN_IF(packed.alloc((size_t)Co2 * C1 * 9 * sizeof(float)));
-        CAMEL_RETURN_IF(pack_weights(w2, packed.f(), Co2, C1, 9));
-        w2p = packed.f();
-    }
-    const int bands = (int)((H - 4) / 2 / CP_BR);
-    const dim3 grid((unsigned)(N * bands), (unsigned)(Co2 / 64));
-    hipLaunchKernelGGL(conv_pair_pool_kernel, grid, dim3(256), 0, stream(), x, w1, b1, w2p, b2, y,
-                       (int)H, (int)Co2, bands, flags1 & (CAMEL_EPI_BIAS | CAMEL_EPI_RELU),
-                       flags2 & (CAMEL_EPI_BIAS | CAMEL_EPI_RELU));
-    const int rc = check_launch("conv_pair_pool_kernel");
-    CAMEL_RETURN_IF(rc);
+    SplitPair p{};
+    p.x = x;
+    p.w1 = w1;
+    p.b1 = b1;
+    p.w2 = w2;
+    p.b2 = b2;
+    p.y = y;
+    p.H = (int)H;
+    p.Co2 = (int)Co2;
+    p.flags1 = flags1 & (CAMEL_EPI_BIAS | CAMEL_EPI_RELU);
+    p.flags2 = flags2 & (CAMEL_EPI_BIAS | CAMEL_EPI_RELU);
+    p.w2_packed = (flags2 & CAMEL_CONV_W_PACKED) != 0;
+    Scratch ws;
+    CAMEL_RETURN_IF(ws.alloc(split_pair_bytes(Co2)));
+    CAMEL_RETURN_IF(split_pair(p, (int)N, ws.p));
     return ok();
 }
 

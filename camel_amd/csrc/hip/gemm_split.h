@@ -74,4 +74,17 @@ SplitConvPlan split_conv_plan(const SplitGemm &g, const SplitConv &c, bool pool,
 // output); `scratch`: weight_bytes + partial_bytes.
 int split_conv(SplitGemm g, SplitConv c, bool quads, bool pool, const SplitConvPlan &plan, void *scratch);
 
+// y = maxpool2x2(conv2(conv1(x))), x [N, 1, H, 28], conv1 1 -> 32 and conv2 32 ->
+// Co2, both 3x3, stride 1, unpadded.
+constexpr int PAIR_C1 = 32;
+struct SplitPair {
+    const float *x, *w1, *b1, *w2, *b2;
+    float *y;
+    int H, Co2, bands; // bands: set by split_pair
+    int flags1, flags2, w2_packed;
+};
+bool split_pair_serves(int64_t H, int64_t W, int64_t C1, int64_t Co2);
+size_t split_pair_bytes(int64_t Co2); // scratch for conv2's split weights
+int split_pair(SplitPair p, int N, void *scratch);
+
 } // namespace camel_hip

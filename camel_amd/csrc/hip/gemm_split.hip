@@ -393,43 +393,44 @@ __device__ __forceinline__ void store_conv(const SplitGemm &g, const SplitConv &
 
 // The sums of a tile that the split cannot form: all of them where an operand
 // was below its range (flag bit TINY_SEEN), the non-finite ones otherwise, in
-// fp32 (v_mfma_f32_16x16x4_f32, the same result layout), 4 columns of blocks at
-// a time.  a(i, k), b(j, k): this lane's operand of block row i, column j.
+// fp32 (v_mfma_f32_16x16x4_f32, the same result layout), a few columns of
+// blocks at a time.  a(i, k), b(j, k): this lane's operand of block row i, column j.
 enum { TINY_SEEN = 1, NOT_FINITE = 2 };
 template <int FM, int FN, class A, class B>
 __device__ __forceinline__ void fp32_sums(f4 (*acc)[FN], int kbeg, int kend, bool all, int oct, A a, B b) {
-    static_assert(FN % 4 == 0, "columns in fours");
+    constexpr int JW = FN % 4 == 0 ? 4 : 2;
+    static_assert(FN % JW == 0, "columns in groups");
     auto sums = [&](int j0, auto &y, int jy) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) y[i][jy + j] = f4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < JW; ++j) y[i][jy + j] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
         for (int k0 = kbeg; k0 < kend; k0 += 4) {
             const int k = k0 + oct;
-            float fa[FM], fb[4];
+            float fa[FM], fb[JW];
 #pragma unroll
             for (int i = 0; i < FM; ++i) fa[i] = k < kend ? a(i, k) : 0.f;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) fb[j] = k < kend ? b(j0 + j, k) : 0.f;
+            for (int j = 0; j < JW; ++j) fb[j] = k < kend ? b(j0 + j, k) : 0.f;
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+                for (int j = 0; j < JW; ++j)
                     y[i][jy + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j], fa[i], y[i][jy + j], 0, 0, 0);
         }
     };
 #pragma unroll
-    for (int j0 = 0; j0 < FN; j0 += 4) {
+    for (int j0 = 0; j0 < FN; j0 += JW) {
         if constexpr (FM * FN > 16) { // no registers for both: all of them
             sums(j0, acc, j0);
         } else {
-            f4 y[FM][4];
+            f4 y[FM][JW];
             sums(j0, y, 0);
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+                for (int j = 0; j < JW; ++j)
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
                         if (all || !(__builtin_fabsf(acc[i][j0 + j][v]) < INFINITY)) acc[i][j0 + j][v] = y[i][j][v];
@@ -644,6 +645,226 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, 
     tile.N = nend;
     tile.partial = nullptr;
     store_conv<T::FM, T::FN, POOL>(tile, c, acc, 0, mw, nw + 4 * oct);
+}
+
+// ---- the first two convolutions of an image CNN, fused with the pool -----------
+//
+// y = maxpool2x2(conv2(conv1(x))) (each conv with its optional bias and relu)
+// for a one-channel input: conv1 1 -> PAIR_C1 channels, 3x3, then conv2 PAIR_C1
+// -> Co2, 3x3, both stride 1 and unpadded, then the 2x2 stride-2 pool.  conv1's
+// output (PAIR_C1 x 26 x 26 per 28 x 28 image, 44 MB at batch 512) never
+// reaches HBM: a work-group computes the rows of it that its band of conv2
+// rows reads, splits them into LDS as the patch kernel's chunks, and multiplies
+// all nine taps from there.
+//   * work-group = (image, band of PAIR_BR pooled rows = 2 PAIR_BR conv2 rows) x
+//     64 output channels; 4 waves as 2 (channels) x 2 (column halves) of 2 x 6
+//     blocks; columns in pool order, a window per lane quad of results, 16
+//     columns a 2 x 2 block of windows (pair_window);
+//   * conv1: a wave an octet of channels, a lane a pixel, the weights scalar;
+//     the direct kernel's FMA chain (k ascending, then bias and x * (x > 0)), so
+//     the patch splits exactly the values the conv1 kernel stores;
+//   * the MFMA sequence and the epilogue are those of the pooled split
+//     convolution of 32 channels, so the result equals the two conv calls and
+//     the pool bit for bit.
+// The 16 pixels of 16 columns, (2 py + r, 2 px + c) for r, c in 0..3, lie on 16
+// chunks that differ mod 16 at a row pitch of 28 (28 r = 0, 12, 8, 4 mod 16):
+// no bank conflicts.  CNN forward at batch 512: 119.0 us with the pair in fp32
+// MFMA (98 us of it), 78.6 us so.
+constexpr int PAIR_W = 28, PAIR_OW1 = PAIR_W - 2, PAIR_PW = (PAIR_OW1 - 2) / 2;
+constexpr int PAIR_BR = 4;                     // pooled rows per work-group
+constexpr int PAIR_R1 = 2 * PAIR_BR + 2;       // conv1 rows a band reads
+constexpr int PAIR_IR = PAIR_R1 + 2;           // input rows a band reads
+constexpr int PAIR_POS = PAIR_R1 * PAIR_W;     // chunk positions of a plane (row pitch 28)
+constexpr int PAIR_COLS = PAIR_BR * PAIR_PW * 4;
+constexpr int PAIR_FN = PAIR_COLS / 32;        // column blocks per wave
+static_assert(PAIR_W % 16 == 12, "conflict-free patch row pitch");
+static_assert(PAIR_COLS % 32 == 0 && PAIR_BR % 2 == 0 && PAIR_PW % 2 == 0, "windows in 2 x 2 blocks");
+
+// The pool window (row py of the band, column px) of GEMM column col.
+__device__ __forceinline__ void pair_window(int col, int &py, int &px) {
+    const int g = col >> 4, w4 = (col >> 2) & 3;
+    py = 2 * (g / (PAIR_PW / 2)) + (w4 >> 1);
+    px = 2 * (g % (PAIR_PW / 2)) + (w4 & 1);
+}
+
+// conv1's finished value from its 9 inputs.
+__device__ __forceinline__ float pair_conv1(const float *x, const float *w, float bias, bool has_bias,
+                                            bool has_relu) {
+    float v = 0.f;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) v = __builtin_fmaf(w[k], x[k], v);
+    if (has_bias) v = v + bias;
+    if (has_relu) v = relu_idiom(v);
+    return v;
+}
+
+__global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4 *w2_split) {
+    constexpr int FM = 2, FN = PAIR_FN;
+    __shared__ u4 patch[12 * PAIR_POS];
+    __shared__ __attribute__((aligned(16))) float img[PAIR_IR * PAIR_W];
+    __shared__ uint32_t flag;
+    const bool bias1 = p.flags1 & CAMEL_EPI_BIAS, relu1 = p.flags1 & CAMEL_EPI_RELU;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1, r16 = lane & 15, oct = lane >> 4;
+    const int n = blockIdx.x / p.bands, band = blockIdx.x - n * p.bands;
+    const int m0 = blockIdx.y * 64, PH = p.bands * PAIR_BR;
+    const int Y0 = band * 2 * PAIR_BR; // first conv2 (and conv1) row of the band
+    const float *xi = p.x + ((size_t)n * p.H + Y0) * PAIR_W;
+    const int a_blocks = p.Co2 / 16;
+    const u4 *a_src[FM];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) a_src[i] = w2_split + (size_t)(m0 / 16 + wm * FM + i) * 192 + lane;
+    u4 an[FM][3];
+    auto load_a = [&](int tap) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) an[i][q] = a_src[i][(size_t)tap * a_blocks * 192 + 64 * q];
+    };
+    load_a(0);
+    if (tid == 0) flag = 0;
+    // The band's input rows, 16 bytes per thread (zeros past the image: never
+    // read by a valid output).
+    if (tid < PAIR_IR * PAIR_W / 4) {
+        const int r = Y0 + tid / (PAIR_W / 4);
+        reinterpret_cast<f4 *>(img)[tid] =
+            r < p.H ? reinterpret_cast<const f4 *>(xi)[tid] : f4{0.f, 0.f, 0.f, 0.f};
+    }
+    __syncthreads();
+    us2 tiny = {0xffff, 0xffff};
+    const float *w1 = p.w1 + 8 * wave * 9;
+#pragma unroll 1
+    for (int q = lane; q < PAIR_POS; q += 64) {
+        const int r = q / PAIR_W, c = min(q - r * PAIR_W, PAIR_OW1 - 1); // the pitch's last two repeat
+        float xv[9], f[8];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) xv[k] = img[(r + k / 3) * PAIR_W + c + k % 3];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            f[e] = pair_conv1(xv, w1 + 9 * e, bias1 ? p.b1[8 * wave + e] : 0.f, bias1, relu1);
+        u4 d[3];
+        split8(f, d, tiny);
+#pragma unroll
+        for (int h = 0; h < 3; ++h) patch[(h * 4 + wave) * PAIR_POS + q] = d[h];
+    }
+    __syncthreads();
+
+    int at[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        const int col = (wn * FN + j) * 16 + r16, d = col & 3;
+        int py, px;
+        pair_window(col, py, px);
+        at[j] = oct * PAIR_POS + (2 * py + (d >> 1)) * PAIR_W + 2 * px + (d & 1);
+    }
+    f4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    bf8 b[2][3], a[FM][3];
+    f4 t[2][FM];
+    auto fetch = [&](int j, int off, bf8 *d) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) d[q] = __builtin_bit_cast(bf8, patch[q * 4 * PAIR_POS + at[j] + off]);
+    };
+    fetch(0, 0, b[0]);
+    constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll 1
+    for (int kh = 0; kh < 3; ++kh) {
+#pragma unroll
+        for (int kw = 0; kw < 3; ++kw) {
+            const int off = kh * PAIR_W + kw, next = kw < 2 ? off + 1 : min(kh + 1, 2) * PAIR_W;
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+#pragma unroll
+                for (int q = 0; q < 3; ++q) a[i][q] = __builtin_bit_cast(bf8, an[i][q]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) note_tiny(an[i][0][e], tiny);
+            }
+            load_a(min(3 * kh + kw + 1, 8));
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const int u = (kw * FN + j) & 1;
+                fetch((j + 1) % FN, j + 1 < FN ? off : next, b[u ^ 1]);
+#pragma unroll
+                for (int i = 0; i < FM; ++i) t[u][i] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int q = 0; q < 6; ++q)
+#pragma unroll
+                    for (int i = 0; i < FM; ++i)
+                        t[u][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[u][PB[q]], a[i][PA[q]], t[u][i], 0,
+                                                                          0, 0);
+                if (j > 0)
+#pragma unroll
+                    for (int i = 0; i < FM; ++i) acc[i][j - 1] += t[u ^ 1][i];
+#pragma unroll
+                for (int r = 0; r < 6 * FM; ++r) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    if (r % FM == FM - 1 && r < 3 * FM) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    if (r >= FM) __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int i = 0; i < FM; ++i) acc[i][FN - 1] += t[(kw * FN + FN - 1) & 1][i];
+        }
+    }
+
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
+    if (bad) atomicOr(&flag, (uint32_t)NOT_FINITE);
+    if (tiny.x < TINY || tiny.y < TINY) atomicOr(&flag, (uint32_t)TINY_SEEN);
+    __syncthreads();
+    if (flag) {
+        SplitGemm g2{};
+        SplitConv c2{};
+        g2.A = p.w2;
+        c2.C = c2.unit = PAIR_C1;
+        c2.taps = 9;
+        c2.w_packed = p.w2_packed;
+        fp32_sums<FM, FN>(
+            acc, 0, 9 * PAIR_C1, flag & TINY_SEEN, oct,
+            [&](int i, int k) { return conv_weight(g2, c2, m0 + (wm * FM + i) * 16 + r16, k); },
+            [&](int j, int k) {
+                const int col = (wn * FN + j) * 16 + r16, d = col & 3, tap = k / PAIR_C1, ch = k % PAIR_C1;
+                int py, px;
+                pair_window(col, py, px);
+                const int r = 2 * py + (d >> 1) + tap / 3, c = 2 * px + (d & 1) + tap % 3;
+                float xv[9];
+                for (int e = 0; e < 9; ++e) xv[e] = img[(r + e / 3) * PAIR_W + c + e % 3];
+                return pair_conv1(xv, p.w1 + 9 * ch, bias1 ? p.b1[ch] : 0.f, bias1, relu1);
+            });
+    }
+    // bias, relu, then the window's maximum: first, then strict '>'
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+        const int row = m0 + (wm * FM + i) * 16 + r16;
+        const float bias = (p.flags2 & CAMEL_EPI_BIAS) ? p.b2[row] : 0.f;
+        float *out = p.y + ((size_t)n * p.Co2 + row) * PH * PAIR_PW + (size_t)band * PAIR_BR * PAIR_PW;
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            int py, px;
+            pair_window((wn * FN + j) * 16 + 4 * oct, py, px);
+            f4 v = acc[i][j];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (p.flags2 & CAMEL_EPI_BIAS) v[e] = v[e] + bias;
+                if (p.flags2 & CAMEL_EPI_RELU) v[e] = relu_idiom(v[e]);
+            }
+            float mx = v[0];
+#pragma unroll
+            for (int e = 1; e < 4; ++e)
+                if (v[e] > mx) mx = v[e];
+            out[py * PAIR_PW + px] = mx;
+        }
+    }
 }
 
 // (The conv kernels' first stage below k = 0 is stage 0 of the split weights.)
@@ -1059,6 +1280,9 @@ template <class T> int64_t conv_tiles(const SplitGemm &g) {
 // stages: unsplit 80.)
 int conv_splits(const SplitGemm &g, int64_t tiles, int cus) {
     const int stages = (g.K + BK - 1) / BK;
+    // (Up to 9 stages stay unsplit: the fused pair of first layers, which sums 9
+    // stages in one go, has to match.)
+    if (stages <= 9) return 1;
     int best = 1;
     double best_t = 1e30;
     for (int want = 1; want <= 16; ++want) {
@@ -1246,6 +1470,30 @@ int split_conv(SplitGemm g, SplitConv c, bool quads, bool pool, const SplitConvP
                      : launch_conv<C64, false>(g, c, pool, plan.splits, partial);
     return quads ? launch_conv<C128, true>(g, c, pool, plan.splits, partial)
                  : launch_conv<C128, false>(g, c, pool, plan.splits, partial);
+}
+
+bool split_pair_serves(int64_t H, int64_t W, int64_t C1, int64_t Co2) {
+    return W == PAIR_W && C1 == PAIR_C1 && Co2 > 0 && Co2 % 64 == 0 && H >= 6 && (H - 4) % (2 * PAIR_BR) == 0;
+}
+
+size_t split_pair_bytes(int64_t Co2) { return (size_t)9 * (Co2 / 16) * 3072; }
+
+int split_pair(SplitPair p, int N, void *scratch) {
+    SplitGemm g{};
+    SplitConv c{};
+    g.A = p.w2;
+    g.M = p.Co2;
+    g.K = 9 * PAIR_C1;
+    c.C = c.unit = PAIR_C1;
+    c.taps = 9;
+    c.w_packed = p.w2_packed;
+    u4 *w2 = static_cast<u4 *>(scratch);
+    hipLaunchKernelGGL(split_weights_kernel, dim3(9, p.Co2 / 16), dim3(64), 0, stream(), g, c, w2);
+    CAMEL_RETURN_IF(check_launch("split_weights_kernel"));
+    p.bands = (p.H - 4) / 2 / PAIR_BR;
+    hipLaunchKernelGGL(conv_pair_kernel, dim3((unsigned)(N * p.bands), (unsigned)(p.Co2 / 64)), dim3(256), 0,
+                       stream(), p, w2);
+    return check_launch("conv_pair_kernel");
 }
 
 } // namespace camel_hip
