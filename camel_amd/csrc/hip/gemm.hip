@@ -3092,7 +3092,7 @@ SgemmPlan plan_sgemm(const GemmArgs &g, bool atrans) {
     int bk = 0;
     const int cus = device_cu_count();
     if (g.M > 32) {
-        p.split = split_gemm_plan(g.M, g.N, g.K, atrans || !p.avec || !p.bvec, g.lda, g.ldb, cus);
+        p.split = split_gemm_plan(g.M, g.N, g.K, atrans, !p.avec, !p.bvec, g.lda, g.ldb, cus);
         if (p.split.tile != SplitTile::None) {
             p.path = SgemmPath::Split;
             p.partial_bytes = p.split.partial_bytes;

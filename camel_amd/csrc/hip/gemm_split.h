@@ -42,7 +42,7 @@ struct SplitConv {
 };
 
 // How the split kernels run a GEMM: the tile and the K splits.
-enum class SplitTile { None, T256, T128 };
+enum class SplitTile { None, T256, T128, T64 };
 struct SplitPlan {
     SplitTile tile = SplitTile::None;
     int splits = 1;
@@ -51,9 +51,9 @@ struct SplitPlan {
 
 // The plan for C[M, N] = A[M, K] B[K, N]; SplitTile::None where the fp32 MFMA
 // kernels are faster or the kernels' 32-bit offsets do not reach.
-// `unaligned`: A transposed or an operand without 16-byte aligned rows.
-SplitPlan split_gemm_plan(int64_t M, int64_t N, int64_t K, bool unaligned, int64_t lda, int64_t ldb,
-                          int cus);
+// `a_unaligned`, `b_unaligned`: an operand without 16-byte aligned rows.
+SplitPlan split_gemm_plan(int64_t M, int64_t N, int64_t K, bool a_trans, bool a_unaligned, bool b_unaligned,
+                          int64_t lda, int64_t ldb, int cus);
 // Runs it on the library stream; `partial`: plan.partial_bytes of scratch.
 int split_gemm(SplitGemm g, bool a_trans, const SplitPlan &plan, float *partial);
 

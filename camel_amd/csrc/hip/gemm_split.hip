@@ -1014,7 +1014,15 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
     __syncthreads();
     const int b_rd = oct * T::BN + wn * T::FN * 16 + r16;
     bf8 b[2][3];
-    f4 t[2][T::FM];
+    // A wave of one block row runs its six products as two chains, so that no
+    // MFMA waits for the one before.
+    constexpr int NC = T::FM == 1 ? 2 : 1;
+    f4 t[2][T::FM * NC];
+    auto add_t = [&](int j) {
+#pragma unroll
+        for (int i = 0; i < T::FM; ++i)
+            acc[i][j] += NC == 2 ? t[j & 1][i] + t[j & 1][i + NC - 1] : t[j & 1][i];
+    };
     auto fetch = [&](const u4 *Bs, int j, bf8 *d) {
 #pragma unroll
         for (int q = 0; q < 3; ++q)
@@ -1047,16 +1055,15 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
             // barrier in the one before)
             fetch(j + 1 < T::FN ? Bc : Bn, (j + 1) % T::FN, b[(j + 1) & 1]);
 #pragma unroll
-            for (int i = 0; i < T::FM; ++i) t[j & 1][i] = f4{0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < T::FM * NC; ++i) t[j & 1][i] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int p = 0; p < 6; ++p)
 #pragma unroll
-                for (int i = 0; i < T::FM; ++i)
-                    t[j & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j & 1][PB[p]], a[i][PA[p]],
-                                                                          t[j & 1][i], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < T::FM; ++i)
-                if (j > 0) acc[i][j - 1] += t[(j + 1) & 1][i];
+                for (int i = 0; i < T::FM; ++i) {
+                    f4 &c = t[j & 1][i + p % NC];
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j & 1][PB[p]], a[i][PA[p]], c, 0, 0, 0);
+                }
+            if (j > 0) add_t(j - 1);
             if (j == J_ST) {
                 store_b(Bn, rb);
                 load_b(k2, rb);
@@ -1113,8 +1120,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
             split_a(ra);
             load_all_a(k2, ra);
         }
-#pragma unroll
-        for (int i = 0; i < T::FM; ++i) acc[i][T::FN - 1] += t[(T::FN - 1) & 1][i];
+        add_t(T::FN - 1);
     }
 
     bool bad = false;
@@ -1225,10 +1231,13 @@ __global__ __launch_bounds__(256) void split_conv_reduce_kernel(SplitGemm g, Spl
     }
 }
 
-// 256 x 256: 8 waves of 32 x 256.  128 x 128: 8 waves, 4 of 32 x 128 on each of
-// two k groups.
+// 256 x 256: 8 waves of 32 x 256.  128 x 128 and 64 x 64: 8 waves, 4 of 32 x 128
+// or 16 x 64 on each of two k groups (64 x 64 with the six products of a block
+// as two MFMA chains: 21.1 -> 20.2 us at 1024^3, 14.1 -> 14.5 at 68 x 192 x
+// 8021; four k groups of two 32 x 64 waves: 300 x 3000 x 800 18.8 -> 20.6).
 using T256 = STile<2, 16, 8, 1, 1>;
 using T128 = STile<2, 8, 4, 1, 2>;
+using T64 = STile<1, 4, 4, 1, 2>;
 
 // Convolutions: 4 waves of 32 channels x 128 pixels (two work-groups share a
 // CU, so one's first loads and stores overlap the other's products), 2 x 2 of
@@ -1366,50 +1375,93 @@ int launch_conv(SplitGemm g, const SplitConv &c, bool pool, int splits, float *p
 
 } // namespace
 
-// The rule: microseconds of each (tile, splits) choice against those of the fp32
-// MFMA kernels, from the sizes alone.  A split work-group takes a fixed time
-// (prologue, tail, launch) plus one per step; partials are written and read
-// at about 6 TB/s after a reduce launch.  The constants are fits to measured
-// calls (start of this kernel / fp32 kernels / estimate, us): 4096^3 538 / 964
-// / 533, 1000 x 3001 x 2047 88 / 162 / 87, 1024 x 1024 x 8192 transposed 95 /
-// 193 / 99, 2048^3 95 / 131 / 97, 1500^3 60 / 86 / 59, 128 x 4096 x 4096 39 /
-// 44 / 37; and 1024^3 32 / 21 / 26, 600^3 23 / 15, 512^3 19 / 12, which stay on
-// the fp32 kernels: their 64 x 64 tiles fill the chip without partials, and a
-// 64 x 64 split tile converts each value too often (22.8 us at 1024^3).
-SplitPlan split_gemm_plan(int64_t M, int64_t N, int64_t K, bool unaligned, int64_t lda, int64_t ldb,
-                          int cus) {
+// Microseconds of a product on the fp32 MFMA kernels, as their plan chooses the
+// tile (256 and 128 where these fill the CUs, else 64, or 32 where 64 covers
+// less than half of them) and the K splits.  Constants: least squares over 260
+// measured shapes of 64..7900 rows and columns, k 64..7400 (7% rms).
+static double fp32_us(int64_t M, int64_t N, int64_t K, bool at, bool ua, bool ub, int cus) {
+    auto up = [](int64_t v, int64_t m) { return (v + m - 1) / m; };
+    auto tiles = [&](int64_t edge) { return up(M, edge) * up(N, edge); };
+    const double out = 4.0 * M * N / 5e6; // C's bytes
+    const bool plain = !at && !ua && !ub;
+    if (tiles(256) >= cus)
+        return up(tiles(256), cus) * up(K, 64) * (plain ? 14.7 : 16.0) + out;
+    if (tiles(128) >= cus)
+        return 4 + up(tiles(128), cus) * up(K, 64) * (plain ? 3.7 : 4.2) + 2 * out;
+    auto splits_of = [&](int64_t t) {
+        return std::max<int64_t>(1, std::min<int64_t>(up(cus, t), std::min<int64_t>(K / 256, 64)));
+    };
+    int64_t edge = 64, splits = tiles(64) >= cus ? 1 : splits_of(tiles(64));
+    if (tiles(64) * splits * 2 < cus) {
+        edge = 32;
+        splits = splits_of(tiles(32));
+    }
+    const int64_t wgs = tiles(edge) * splits, steps = up(up(K, 64), splits), rounds = up(wgs, cus);
+    const double part = splits > 1 ? 8.0 * splits * M * N / 6e6 : 0.0; // partials, written and read
+    if (edge == 32)
+        return 2.6 + steps * std::max(1.0, (double)wgs / cus) * (0.65 + 0.2 * at + 0.2 * ub) +
+               (plain ? 0 : 1.3) + (splits > 1 ? 2.5 : 0.0) + 3 * part + 2.5 * out;
+    return 4 + steps * rounds * ((plain ? 1.08 : rounds == 1 ? 1.5 : 1.12) + 0.2 * at + 0.2 * ua + 0.2 * ub) +
+           (splits > 1 ? 0.9 : 0.0) + 2.3 * part + 1.4 * out;
+}
+
+// The rule: the (tile, K splits) of the shortest estimate, if it is below 0.9 of
+// the fp32 kernels' (the margin covers the fits' error).  A work-group takes a
+// fixed time (prologue, tail, launch) plus one per step; partials are written
+// and read at about 6 TB/s after a reduce launch.  128- and 256-edge tiles have
+// a CU to themselves and run in whole rounds; two 64-edge ones share one.
+// Constants: least squares over 1500 measured (shape, tile, splits) (6% rms).
+// Over those shapes the choice is 1.21x the fp32 kernels and 2% behind the best
+// one.  Sizes enter as whole 64 x 64 tiles, so that a row gives the same bits
+// whether or not its tile is full.  Split / fp32, us: 4096^3 541 / 952, 1000 x 3001 x 2047 80 / 162, 1024 x
+// 1024 x 8192 transposed 96 / 193, 2048^3 90 / 132, 1500^3 61 / 80, 768^3 16 / 23,
+// 300 x 3000 x 800 18 / 27, 68 x 192 x 8021 transposed 14 / 17; and 1024^3 20.5 /
+// 20.5, 512^3 11.5 / 11.6, 256^3 8.1 / 5.0, which stay on the fp32 kernels: one
+// round of tiles whose loads are DMA, where a 64 x 64 split tile converts each
+// value 16 times over, and a classifier head joins the fp32 tile's epilogue.
+SplitPlan split_gemm_plan(int64_t M, int64_t N, int64_t K, bool a_trans, bool a_unaligned, bool b_unaligned,
+                          int64_t lda, int64_t ldb, int cus) {
     SplitPlan best;
     if (K < 64 || lda >= (1 << 21) || ldb >= (1 << 28) || M > INT32_MAX / 512 || N > INT32_MAX / 512)
         return best;
     auto up = [](int64_t v, int64_t m) { return (v + m - 1) / m; };
-    // fp32 kernels: their rate over whole 64 x 64 tiles, lower where an
-    // operand is transposed or its rows are not 16-byte aligned
-    const bool big = up(M, 256) * up(N, 256) >= cus;
-    const double rate = big ? 140e6 : unaligned ? 85e6 : 105e6; // FLOP/us
-    double limit = 0.92 * (3.5 + 2.0 * 64 * up(M, 64) * 64 * up(N, 64) * K / rate);
-    auto consider = [&](SplitTile tile, int edge, int sb, double fixed, double step) {
+    const size_t c_bytes = (size_t)M * N * sizeof(float);
+    M = up(M, 64) * 64;
+    N = up(N, 64) * 64;
+    double limit = 0.9 * fp32_us(M, N, K, a_trans, a_unaligned, b_unaligned, cus);
+    const double out = 4.0 * M * N / 5e6;
+    auto consider = [&](SplitTile tile, int edge, int sb, auto &&estimate) {
         const int64_t tiles = up(M, edge) * up(N, edge);
         if (tiles > INT32_MAX / 64) return;
         for (int want : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32}) {
             const int64_t steps = up(K, sb), per = up(steps, want), used = up(steps, per);
             const size_t bytes = used > 1 ? (size_t)used * M * N * sizeof(float) : 0;
             if (used != want || bytes > CAMEL_HIP_NOALLOC_SCRATCH_BYTES || (want > 1 && per < 4)) continue;
-            const double t = up(tiles * used, cus) * (fixed + step * per) + (used > 1 ? 2.0 + 2.0 * bytes / 6e6 : 0.0);
+            const double t = estimate(tiles * used, (double)per, used > 1, 2.0 * bytes / 6e6);
             if (t < limit) {
                 limit = t;
-                best = {tile, (int)used, bytes};
+                best = {tile, (int)used, used > 1 ? (size_t)used * c_bytes : 0};
             }
         }
     };
-    consider(SplitTile::T256, 256, T256::SB, 8.5, 4.1);
-    consider(SplitTile::T128, 128, T128::SB, 7.0, 2.4);
+    consider(SplitTile::T256, 256, T256::SB, [&](int64_t wgs, double per, bool parts, double bytes) {
+        return up(wgs, cus) * (8.5 + 4.1 * per) + (parts ? 3.6 : 0.0) + 0.9 * bytes;
+    });
+    consider(SplitTile::T128, 128, T128::SB, [&](int64_t wgs, double per, bool parts, double bytes) {
+        return up(wgs, cus) * (8.9 + 2.06 * per) + (parts ? 3.6 : 0.0) + 0.9 * bytes + 1.1 * out;
+    });
+    consider(SplitTile::T64, 64, T64::SB, [&](int64_t wgs, double per, bool parts, double bytes) {
+        const double share = wgs <= cus ? 1.0 : std::max(1.6, 0.15 + (double)wgs / cus);
+        return 4.4 + per * share * (0.88 + 0.18 * a_trans) + (parts ? 2.7 : 0.0) + 1.55 * bytes + 2.5 * out;
+    });
     return best;
 }
 
 int split_gemm(SplitGemm g, bool a_trans, const SplitPlan &plan, float *partial) {
     g.partial = partial;
     if (plan.tile == SplitTile::T256) return launch<T256>(g, a_trans, plan.splits);
-    return launch<T128>(g, a_trans, plan.splits);
+    if (plan.tile == SplitTile::T128) return launch<T128>(g, a_trans, plan.splits);
+    return launch<T64>(g, a_trans, plan.splits);
 }
 
 bool split_conv_serves(int64_t N, int64_t C, int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW,

@@ -23,6 +23,9 @@ SHAPES = [
     (129, 4096, 2048, False),   # 128x128, two k groups, one row in the last tile row
     (8192, 512, 500, False),    # 128x128 unsplit, K % 64 = 52
     (321, 333, 8190, True),     # 128x128 with many K splits, everything odd
+    (300, 3000, 800, False),    # 64x64, last row tile 44, last column tile 56, K % 64 = 32
+    (67, 201, 8021, True),      # 64x64 with many K splits, everything odd
+    (2662, 553, 409, False),    # 64x64, more tiles than CUs, rows unaligned
 ]
 
 
@@ -105,7 +108,7 @@ def test_operands_outside_the_exact_range(M, N, Kd, trans):
     assert np.all(np.abs(got - ref) <= lim)
 
 
-@pytest.mark.parametrize("M,N,Kd,trans", SHAPES[:4])
+@pytest.mark.parametrize("M,N,Kd,trans", SHAPES[:4] + SHAPES[6:8])
 def test_special_values_propagate(M, N, Kd, trans):
     print(f"split special {M}x{N}x{Kd}", flush=True)
     rng = np.random.default_rng(M + 13 * Kd)
