@@ -9,8 +9,9 @@
 //                                   here, within 1 ulp of the fp64 libm exp)
 //   s  = fl32(sum_j double(e_j))   (tensorSumAxis 887-922, fp64 accumulation)
 //   y  = fl32(e / s)               (divide, bit-exact through 1/s in fp64)
-// One wave owns one row; rows up to 64*4*ITEMS columns stay in registers, so
-// HBM sees one read and one write per element (8 B/elem).  The fp64 sum
+// One wave owns one row, several short rows share one, and long rows take a
+// work-group; rows up to 32768 columns stay in registers, so HBM sees one read
+// and one write per element (8 B/elem).  The fp64 sum
 // differs from the reference's sequential order only in the last bits of
 // the double, below the fp32 rounding of s.
 //
@@ -26,6 +27,7 @@ namespace camel_hip {
 namespace {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4))); // 16-byte access, 4-byte aligned
 
 constexpr int WAVE = 64;
 
@@ -117,25 +119,182 @@ __global__ __launch_bounds__(256) void softmax_rows_kernel(const float *__restri
         softmax_row<ITEMS, VEC>(x + row * cols, y + row * cols, cols, lane);
 }
 
-// Rows longer than the register budget: max pass, sum pass, write pass.
-__global__ __launch_bounds__(256) void softmax_rows_long_kernel(const float *__restrict__ x,
-                                                                float *__restrict__ y,
-                                                                int64_t rows, int64_t cols) {
+// Short rows: a wave takes 64 >> LG rows at once, 1 << LG lanes per row, one
+// float4 (VEC) or one value per lane, SHORT_ROWS such groups in flight.  The
+// sums of a row are added in the order of the one-row kernel, whose further
+// lanes add exact zeros.
+constexpr int SHORT_ROWS = 4;
+
+template <int LG, bool VEC>
+__global__ __launch_bounds__(256) void softmax_short_rows_kernel(const float *__restrict__ x,
+                                                                 float *__restrict__ y, int64_t rows,
+                                                                 int cols) {
+    constexpr int NV = VEC ? 4 : 1, WIDTH = 1 << LG, PER_WAVE = WAVE >> LG;
     const int lane = threadIdx.x & 63;
-    for (int64_t row = first_row(); row < rows; row += row_step()) {
-    const float *xr = x + row * cols;
-    float *yr = y + row * cols;
-    float m = -INFINITY;
-    for (int64_t c = lane; c < cols; c += WAVE) m = max_gt(m, xr[c]);
+    const int c = (lane & (WIDTH - 1)) * NV;
+    const int64_t chunk = (int64_t)PER_WAVE * SHORT_ROWS;
+    for (int64_t r0 = first_row() * chunk; r0 < rows; r0 += row_step() * chunk) {
+        float v[SHORT_ROWS][NV];
+        int64_t at[SHORT_ROWS];
+        bool in[SHORT_ROWS];
+#pragma unroll
+        for (int u = 0; u < SHORT_ROWS; ++u) {
+            const int64_t row = r0 + u * PER_WAVE + (lane >> LG);
+            at[u] = row * cols + c;
+            in[u] = row < rows && c < cols;
+#pragma unroll
+            for (int i = 0; i < NV; ++i) v[u][i] = -INFINITY;
+            if constexpr (VEC) {
+                if (in[u]) {
+                    const f4 t = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(x + at[u]));
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[u][i] = t[i];
+                }
+            } else if (in[u]) {
+                v[u][0] = x[at[u]];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < SHORT_ROWS; ++u) {
+            float m = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < NV; ++i) m = max_gt(m, v[u][i]);
+#pragma unroll
+            for (int off = WIDTH >> 1; off > 0; off >>= 1) m = max_gt(m, __shfl_xor(m, off));
+            const float x0 = __shfl(v[u][0], 0, WIDTH);
+            if (x0 != x0) m = x0;
+            const float mb = m + 0.0f;
+            double s = 0.0;
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                v[u][i] = softmax_exp(v[u][i], mb);
+                s += (double)v[u][i];
+            }
+#pragma unroll
+            for (int off = WIDTH >> 1; off > 0; off >>= 1) s += __shfl_xor(s, off);
+            const double rcp = 1.0 / (double)(float)s;
+            if (in[u]) {
+                if constexpr (VEC) {
+                    f4 t;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) t[i] = softmax_div(v[u][i], rcp);
+                    __builtin_nontemporal_store(t, reinterpret_cast<f4 *>(y + at[u]));
+                } else {
+                    y[at[u]] = softmax_div(v[u][0], rcp);
+                }
+            }
+        }
+    }
+}
+
+// Block-wide max and sum of a wave's values; every thread gets the result.
+template <int WAVES> __device__ __forceinline__ float block_max_gt(float m, float *lds) {
     m = wave_max_gt(m);
-    const float x0 = xr[0];
-    if (x0 != x0) m = x0;
-    const float mb = m + 0.0f;
-    double s = 0.0;
-    for (int64_t c = lane; c < cols; c += WAVE) s += (double)softmax_exp(xr[c], mb);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = lds[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) m = max_gt(m, lds[w]);
+    return m;
+}
+template <int WAVES> __device__ __forceinline__ double block_sum(double s, double *lds) {
     s = wave_sum(s);
-    const double rcp = 1.0 / (double)(float)s;
-    for (int64_t c = lane; c < cols; c += WAVE) yr[c] = softmax_div(softmax_exp(xr[c], mb), rcp);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
+    __syncthreads();
+    s = lds[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) s += lds[w];
+    return s;
+}
+
+// One work-group per row, the row in registers (ITEMS groups of 4 columns per
+// thread, loaded and stored as 16 bytes also where rows are only 4-byte
+// aligned): rows too long for a wave's registers, and rows too few to fill the
+// chip with one wave each.
+template <int THREADS, int ITEMS, class Quad>
+__global__ __launch_bounds__(THREADS) void softmax_block_kernel(const float *__restrict__ x,
+                                                                float *__restrict__ y, int64_t rows,
+                                                                int cols) {
+    constexpr int WAVES = THREADS / WAVE, NV = ITEMS * 4;
+    __shared__ float lds_max[WAVES];
+    __shared__ double lds_sum[WAVES];
+    const int quads = cols >> 2, tail = cols & 3; // the last `tail` columns belong to quad number `quads`
+    for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+        const float *xr = x + row * cols;
+        float *yr = y + row * cols;
+        float v[NV];
+        const float x0 = xr[0];
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it) {
+            const int q = threadIdx.x + THREADS * it;
+            f4 t = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+            if (q < quads) {
+                t = __builtin_nontemporal_load(reinterpret_cast<const Quad *>(xr + 4 * q));
+            } else if (q == quads) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    if (c < tail) t[c] = xr[4 * q + c];
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[4 * it + c] = t[c];
+        }
+        float m = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) m = max_gt(m, v[j]);
+        m = block_max_gt<WAVES>(m, lds_max);
+        if (x0 != x0) m = x0;
+        const float mb = m + 0.0f;
+        double s = 0.0;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            v[j] = softmax_exp(v[j], mb);
+            s += (double)v[j];
+        }
+        // The next row's max is stored only behind this barrier, and its sum
+        // behind the barrier of that max: no thread still reads the old ones.
+        s = block_sum<WAVES>(s, lds_sum);
+        const double rcp = 1.0 / (double)(float)s;
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it) {
+            const int q = threadIdx.x + THREADS * it;
+            f4 t;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) t[c] = softmax_div(v[4 * it + c], rcp);
+            if (q < quads) {
+                __builtin_nontemporal_store((Quad)t, reinterpret_cast<Quad *>(yr + 4 * q));
+            } else if (q == quads) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    if (c < tail) yr[4 * q + c] = t[c];
+            }
+        }
+    }
+}
+
+// Rows beyond a work-group's registers: max pass, sum pass, write pass.
+constexpr int LONG_THREADS = 1024;
+
+__global__ __launch_bounds__(LONG_THREADS) void softmax_long_kernel(const float *__restrict__ x,
+                                                                    float *__restrict__ y, int64_t rows,
+                                                                    int64_t cols) {
+    constexpr int WAVES = LONG_THREADS / WAVE;
+    __shared__ float lds_max[WAVES];
+    __shared__ double lds_sum[WAVES];
+    for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+        const float *xr = x + row * cols;
+        float *yr = y + row * cols;
+        const float x0 = xr[0];
+        float m = -INFINITY;
+        for (int64_t c = threadIdx.x; c < cols; c += LONG_THREADS) m = max_gt(m, xr[c]);
+        m = block_max_gt<WAVES>(m, lds_max);
+        if (x0 != x0) m = x0;
+        const float mb = m + 0.0f;
+        double s = 0.0;
+        for (int64_t c = threadIdx.x; c < cols; c += LONG_THREADS) s += (double)softmax_exp(xr[c], mb);
+        s = block_sum<WAVES>(s, lds_sum);
+        const double rcp = 1.0 / (double)(float)s;
+        for (int64_t c = threadIdx.x; c < cols; c += LONG_THREADS)
+            yr[c] = softmax_div(softmax_exp(xr[c], mb), rcp);
     }
 }
 
@@ -258,6 +417,30 @@ template <int ITEMS> int launch_softmax(const float *x, float *y, int64_t rows, 
     return check_launch("softmax_rows_kernel");
 }
 
+template <int THREADS, int ITEMS>
+int launch_softmax_block(const float *x, float *y, int64_t rows, int cols, bool vec) {
+    dim3 grid((unsigned)std::min<int64_t>(rows, ROW_GRID_CAP)), block(THREADS);
+    if (vec)
+        hipLaunchKernelGGL((softmax_block_kernel<THREADS, ITEMS, f4>), grid, block, 0, stream(), x, y,
+                           rows, cols);
+    else
+        hipLaunchKernelGGL((softmax_block_kernel<THREADS, ITEMS, f4u>), grid, block, 0, stream(), x, y,
+                           rows, cols);
+    return check_launch("softmax_block_kernel");
+}
+
+template <int LG> int launch_softmax_short(const float *x, float *y, int64_t rows, int cols, bool vec) {
+    if constexpr (LG < 6)
+        if ((1 << LG) * (vec ? 4 : 1) < cols) return launch_softmax_short<LG + 1>(x, y, rows, cols, vec);
+    constexpr int CHUNK = (WAVE >> LG) * SHORT_ROWS;
+    dim3 grid(row_grid((rows + CHUNK - 1) / CHUNK)), block(256);
+    if (vec)
+        hipLaunchKernelGGL((softmax_short_rows_kernel<LG, true>), grid, block, 0, stream(), x, y, rows, cols);
+    else
+        hipLaunchKernelGGL((softmax_short_rows_kernel<LG, false>), grid, block, 0, stream(), x, y, rows, cols);
+    return check_launch("softmax_short_rows_kernel");
+}
+
 int check_axis(int64_t rows, int64_t cols, int64_t &axis, const char *what) {
     if (rows < 0 || cols < 0) return fail(CAMEL_HIP_ERR_SHAPE, std::string(what) + ": negative shape");
     if (!product_fits({rows, cols, 8}, INT64_MAX))
@@ -311,20 +494,43 @@ int camel_hip_softmax_rows(const float *x, float *y, int64_t rows, int64_t cols)
     CAMEL_INIT_OR_RETURN();
     const bool vec = (cols % 4 == 0) && (((uintptr_t)x | (uintptr_t)y) & 15) == 0;
     const int c = (int)cols;
-    if (cols <= 64 * 4)
+    // Up to 4096 columns a wave holds a row.  Short rows share a wave once one
+    // row per wave would queue (262144 x 10: 66 -> 12.6 us, x 64: 82 -> 24; 4096
+    // rows: 3.1 against 4.6, so not below 8192).  A row is spread over a
+    // work-group where rows are too few for the chip (256 x 1024 3.5 -> 2.8 us;
+    // 1024 rows: 3.9 both; 1024 x 2048 5.5 -> 4.9, 4096 rows: 11.8 against 13.1)
+    // or too long for a wave: from 2048 columns on (16384 x 4096 95 -> 85 us, 3001
+    // unaligned columns 113 -> 74, 1024 x 8192 108 -> 10, 4096 x 16384 422 -> 93:
+    // 5.8 TB/s, 4096 x 32768 904 -> 249, 16 x 32768 234 -> 8).  Group sizes: 8
+    // quads per thread beat 4 from 4096 columns on (1024 x 16384: 24.4 us against
+    // 32.2 for 1024 x 4 quads and 25.5 for 256 x 16), whose work-groups of 1024
+    // threads have a CU to themselves.
+    if (cols <= (vec ? 256 : 64) && rows > 8192)
+        CAMEL_RETURN_IF(launch_softmax_short<0>(x, y, rows, c, vec));
+    else if (cols <= 256)
         CAMEL_RETURN_IF(launch_softmax<1>(x, y, rows, c, vec));
-    else if (cols <= 64 * 8)
+    else if (cols <= 512)
         CAMEL_RETURN_IF(launch_softmax<2>(x, y, rows, c, vec));
-    else if (cols <= 64 * 16)
+    else if (cols <= 1024 && rows > 512)
         CAMEL_RETURN_IF(launch_softmax<4>(x, y, rows, c, vec));
-    else if (cols <= 64 * 32)
+    else if (cols <= 1024)
+        CAMEL_RETURN_IF((launch_softmax_block<256, 1>(x, y, rows, c, vec)));
+    else if (cols <= 2048 && rows > 2048)
         CAMEL_RETURN_IF(launch_softmax<8>(x, y, rows, c, vec));
-    else if (cols <= 64 * 64)
-        CAMEL_RETURN_IF(launch_softmax<16>(x, y, rows, c, vec));
+    else if (cols <= 2048)
+        CAMEL_RETURN_IF((launch_softmax_block<256, 2>(x, y, rows, c, vec)));
+    else if (cols <= 4096)
+        CAMEL_RETURN_IF((launch_softmax_block<256, 4>(x, y, rows, c, vec)));
+    else if (cols <= 8192)
+        CAMEL_RETURN_IF((launch_softmax_block<256, 8>(x, y, rows, c, vec)));
+    else if (cols <= 16384)
+        CAMEL_RETURN_IF((launch_softmax_block<512, 8>(x, y, rows, c, vec)));
+    else if (cols <= 32768)
+        CAMEL_RETURN_IF((launch_softmax_block<1024, 8>(x, y, rows, c, vec)));
     else {
-        hipLaunchKernelGGL(softmax_rows_long_kernel, dim3(row_grid(rows)), dim3(256), 0,
-                           stream(), x, y, rows, cols);
-        CAMEL_RETURN_IF(check_launch("softmax_rows_long_kernel"));
+        hipLaunchKernelGGL(softmax_long_kernel, dim3((unsigned)std::min<int64_t>(rows, ROW_GRID_CAP)),
+                           dim3(LONG_THREADS), 0, stream(), x, y, rows, cols);
+        CAMEL_RETURN_IF(check_launch("softmax_long_kernel"));
     }
     return ok();
 }
