@@ -1648,27 +1648,56 @@ int launch_thin(const float *A, const float *B, float *C, int M, int N, int K, c
 //     overlaps (16 x 4096 x 4096: 16.07 -> 15.31 us per call);
 //   * the 8 waves' sums meet in LDS in wave order; thread x then owns row
 //     x / 16 and 4 consecutive columns, so the results (or the partials of
-//     work-groups along K, [ks][M][N], which skinny_reduce_kernel sums in ks
-//     order before the epilogue) leave as one 16-byte store per thread.
+//     work-groups along K, [ks][M][N rounded up to 4], which
+//     skinny_reduce_kernel sums in ks order before the epilogue) leave as one
+//     16-byte store per thread.
 //     Letting the last work-group of a strip add the partials needs
 //     device-scope release/acquire fences, and on this chip each one writes
 //     back or invalidates an XCD's whole L2: measured several times slower.
-// Work-groups whose rows, columns or k run past the operands take the same
-// loop with guarded scalar loads (a guarded load compiles to a branch, after
-// which the compiler waits for all loads at once, so full work-groups keep
-// the guard-free path).
+// Rows past M repeat the last one and the last column group starts at N - 4 (a
+// row or column of an MFMA reaches no other one, and neither is stored), and
+// 16-byte loads need 4-byte alignment only, so every M, N >= 4 and alignment
+// takes the guard-free loads; a work-group whose k run past K clamps its
+// addresses and zeroes both operands with selects.  (A guarded load compiles
+// to a branch, after which the compiler waits for all loads at once: with M <
+// 16 on guarded loads 1 x 4096 x 4096 took 16.7 us, 14.4 without; 17 rows 21.7,
+// 17.4.  N % 4 != 0, on 32 x 128 tiles against here: 16 x 3001 x 2047 18.4 and
+// 12.1, 7 x 1001 x 77 7.7 and 4.0, 12 x 5 x 3000 16.9 and 6.7, 32 x 8191 x 8192
+// 78.5 and 69.6.)
 constexpr int SK_WAVES = 8;
 constexpr int SK_COLS = 64;
 constexpr int SK_STEPS = 4;                          // 4-row MFMA steps per chunk and wave
 constexpr int SK_CHUNK = SK_WAVES * 4 * SK_STEPS;    // k rows per chunk of the work-group
 constexpr int SK_MAX_KGROUPS = 65535;                // grid.y limit
 
+// Bias, relu and the store of the column group of `row` at ocol: the columns
+// min(ocol, N - 4) .. +3, of which those below ocol are the group before's.
+__device__ __forceinline__ void skinny_store(float *C, int row, int ocol, int N, float *v,
+                                             const float *bias, int flags) {
+    typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+    const int col = min(ocol, N - 4);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        if (flags & CAMEL_EPI_BIAS) v[c] = v[c] + bias[col + c];
+        if (flags & CAMEL_EPI_RELU) v[c] = relu_idiom(v[c]);
+    }
+    float *out = C + (size_t)row * N + col;
+    if (col == ocol)
+        *reinterpret_cast<floatx4u *>(out) = floatx4u{v[0], v[1], v[2], v[3]};
+    else
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (col + c >= ocol) out[c] = v[c];
+}
+
 template <int MT, int CH>
 __global__ __launch_bounds__(SK_WAVES * 64) void sgemm_skinny_kernel(
     const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, int M, int N,
-    int K, const float *__restrict__ bias, int flags, float *__restrict__ partial, int a_vec) {
+    int K, const float *__restrict__ bias, int flags, float *__restrict__ partial) {
     typedef float floatx4 __attribute__((ext_vector_type(4)));
+    typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
     constexpr int S = SK_STEPS, KR = SK_CHUNK * CH;
+    static_assert(S == 4, "a lane's k of a chunk are one 16-byte load of A");
     __shared__ float4 red[SK_WAVES][MT * 4][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, q = lane >> 4;
@@ -1676,68 +1705,63 @@ __global__ __launch_bounds__(SK_WAVES * 64) void sgemm_skinny_kernel(
     const int n0 = strip * SK_COLS;
     const int kb0 = ks * KR;
     const int krow0 = kb0 + wave * 4 * S + q * S; // lane's first k of chunk 0
-    const int col = n0 + 4 * r16;
+    const int col = min(n0 + 4 * r16, N - 4);
 
     floatx4 acc[MT][4];
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
         for (int c = 0; c < 4; ++c) acc[t][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const float *arow[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) arow[t] = A + (size_t)min(16 * t + r16, M - 1) * K;
 
     auto stream_k = [&](auto full_tag) {
         constexpr bool FULL = decltype(full_tag)::value;
-        floatx4 b[S];
-        float4 a[MT][S / 4];
+        floatx4 b[S], a[MT];
         auto load = [&](int c) {
-            const int kc = krow0 + c * SK_CHUNK;
+            const int k = krow0 + c * SK_CHUNK;
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                const int row = 16 * t + r16;
+                if (FULL) {
+                    a[t] = *reinterpret_cast<const floatx4u *>(arow[t] + k);
+                } else {
 #pragma unroll
-                for (int j = 0; j < S / 4; ++j) {
-                    const int k = kc + 4 * j;
-                    if (FULL) {
-                        a[t][j] = *reinterpret_cast<const float4 *>(A + (size_t)row * K + k);
-                    } else {
-                        float e[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            e[i] = (row < M && k + i < K) ? A[(size_t)row * K + k + i] : 0.f;
-                        a[t][j] = make_float4(e[0], e[1], e[2], e[3]);
+                    for (int i = 0; i < 4; ++i) {
+                        const float e = arow[t][min(k + i, K - 1)];
+                        a[t][i] = k + i < K ? e : 0.f;
                     }
                 }
             }
 #pragma unroll
             for (int s = 0; s < S; ++s) {
-                const int k = kc + s;
-                b[s] = (FULL || (col < N && k < K))
-                           ? __builtin_nontemporal_load(
-                                 reinterpret_cast<const floatx4 *>(B + (size_t)k * N + col))
-                           : floatx4{0.f, 0.f, 0.f, 0.f};
+                const int ks = FULL ? k + s : min(k + s, K - 1);
+                b[s] = __builtin_nontemporal_load(reinterpret_cast<const floatx4u *>(B + (size_t)ks * N + col));
+                if (!FULL)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) b[s][i] = k + s < K ? b[s][i] : 0.f;
             }
         };
         auto multiply = [&]() {
 #pragma unroll
             for (int s = 0; s < S; ++s)
 #pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    const float4 a4 = a[t][s / 4];
-                    const float av = (s % 4 == 0) ? a4.x : (s % 4 == 1) ? a4.y : (s % 4 == 2) ? a4.z : a4.w;
-                    acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b[s][0], acc[t][0], 0, 0, 0);
-                    acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b[s][1], acc[t][1], 0, 0, 0);
-                    acc[t][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b[s][2], acc[t][2], 0, 0, 0);
-                    acc[t][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b[s][3], acc[t][3], 0, 0, 0);
-                }
+                for (int t = 0; t < MT; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][s], b[s][i], acc[t][i], 0, 0, 0);
         };
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
+            // (a chunk past K is zeros)
+            if (!FULL && __builtin_amdgcn_readfirstlane(kb0 + c * SK_CHUNK + wave * 4 * S) >= K) break;
             load(c);
             __builtin_amdgcn_sched_barrier(0);
             multiply();
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    if (a_vec && n0 + SK_COLS <= N && kb0 + KR <= K)
+    if (kb0 + KR <= K)
         stream_k(std::true_type{});
     else
         stream_k(std::false_type{});
@@ -1757,7 +1781,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void sgemm_skinny_kernel(
     if (x >= MT * 256) return;
     const int row = x >> 4, cg = x & 15;
     const int ocol = n0 + 4 * cg;
-    if (row >= M || ocol >= N) return; // N % 4 == 0: a column group is all in or all out
+    if (row >= M || ocol >= N) return;
     const int t = row >> 4, sl = ((row & 15) >> 2) * 16 + cg, e = row & 3;
     float v[4];
 #pragma unroll
@@ -1768,81 +1792,49 @@ __global__ __launch_bounds__(SK_WAVES * 64) void sgemm_skinny_kernel(
         v[c] = s;
     }
     if (nks == 1) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            float y = v[c];
-            if (flags & CAMEL_EPI_BIAS) y = y + bias[ocol + c];
-            if (flags & CAMEL_EPI_RELU) y = relu_idiom(y);
-            v[c] = y;
-        }
-        *reinterpret_cast<float4 *>(C + (size_t)row * N + ocol) = make_float4(v[0], v[1], v[2], v[3]);
+        skinny_store(C, row, ocol, N, v, bias, flags);
         return;
     }
-    // partial layout [ks][M][N]
-    *reinterpret_cast<float4 *>(partial + ((size_t)ks * M + row) * N + ocol) =
+    *reinterpret_cast<float4 *>(partial + ((size_t)ks * M + row) * (4 * ((N + 3) / 4)) + ocol) =
         make_float4(v[0], v[1], v[2], v[3]);
 }
 
 // Sums the skinny kernel's k partials in ks order, then bias and relu; one
-// thread per 4 consecutive outputs of a row (N % 4 == 0).  Small work-groups
-// (SK_REDUCE_THREADS) spread the few outputs over many CUs; the partials are
-// read once, with nontemporal loads.  With `strips` > 0 (N a multiple of
-// SK_COLS), work-group b takes 4 rows of strip b % strips: the skinny
-// kernel's work-groups of that strip (block ids strip + strips * ks) ran on
-// the same XCD when strips % 8 == 0, so the partials are read from that
-// XCD's L2 (16 x 4096 x 4096: 15.30 -> 15.03 us per call); otherwise one
-// thread per float4 in row-major order.
+// thread per column group of a row.  Small work-groups (SK_REDUCE_THREADS)
+// spread the few outputs over many CUs; the partials are read once, with
+// nontemporal loads, up to 8 k groups at a time.  Work-group b takes 4 rows of
+// strip b % strips: the skinny kernel's work-groups of that strip (block ids
+// strip + strips * ks) ran on the same XCD when strips % 8 == 0, so the
+// partials are read from that XCD's L2 (16 x 4096 x 4096: 15.30 -> 15.03 us
+// per call, against one thread per group in row-major order).
 constexpr int SK_REDUCE_THREADS = 64;
-static_assert(SK_REDUCE_THREADS == 4 * SK_COLS / 4, "a strip-mapped work-group is 4 rows of a strip");
+static_assert(SK_REDUCE_THREADS == 4 * SK_COLS / 4, "a work-group is 4 rows of a strip");
 
 __global__ __launch_bounds__(SK_REDUCE_THREADS) void skinny_reduce_kernel(
-    const float4 *__restrict__ partial, float4 *__restrict__ C, int M, int N, int nks,
+    const float4 *__restrict__ partial, float *__restrict__ C, int M, int N, int nks,
     const float *__restrict__ bias, int flags, int strips) {
     typedef float floatx4 __attribute__((ext_vector_type(4)));
-    const size_t total4 = (size_t)M * N / 4;
-    size_t idx;
-    if (strips > 0) {
-        const int strip = blockIdx.x % strips, rows4 = blockIdx.x / strips;
-        const int row = 4 * rows4 + threadIdx.x / (SK_COLS / 4);
-        if (row >= M) return;
-        idx = ((size_t)row * N + (size_t)strip * SK_COLS) / 4 + threadIdx.x % (SK_COLS / 4);
-    } else {
-        idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-        if (idx >= total4) return;
-    }
+    const int strip = blockIdx.x % strips, rows4 = blockIdx.x / strips;
+    const int row = 4 * rows4 + threadIdx.x / (SK_COLS / 4);
+    const int ocol = strip * SK_COLS + 4 * (threadIdx.x % (SK_COLS / 4));
+    if (row >= M || ocol >= N) return;
+    const int groups = (N + 3) / 4;
+    const size_t total4 = (size_t)M * groups, idx = (size_t)row * groups + ocol / 4;
     const floatx4 *p4 = reinterpret_cast<const floatx4 *>(partial);
-    // k groups added in order; their loads go out up to 8 at a time
-    const floatx4 y0 = __builtin_nontemporal_load(p4 + idx);
-    float4 y = make_float4(y0[0], y0[1], y0[2], y0[3]);
+    floatx4 y = __builtin_nontemporal_load(p4 + idx);
     for (int z0 = 1; z0 < nks; z0 += 8) {
         floatx4 p[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u)
             if (z0 + u < nks) p[u] = __builtin_nontemporal_load(p4 + (size_t)(z0 + u) * total4 + idx);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            if (z0 + u < nks) {
-                y.x = y.x + p[u][0];
-                y.y = y.y + p[u][1];
-                y.z = y.z + p[u][2];
-                y.w = y.w + p[u][3];
-            }
-        }
+        for (int u = 0; u < 8; ++u)
+            if (z0 + u < nks)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) y[c] = y[c] + p[u][c];
     }
-    if (flags & CAMEL_EPI_BIAS) {
-        const size_t col = (idx * 4) % (size_t)N;
-        y.x = y.x + bias[col];
-        y.y = y.y + bias[col + 1];
-        y.z = y.z + bias[col + 2];
-        y.w = y.w + bias[col + 3];
-    }
-    if (flags & CAMEL_EPI_RELU) {
-        y.x = relu_idiom(y.x);
-        y.y = relu_idiom(y.y);
-        y.z = relu_idiom(y.z);
-        y.w = relu_idiom(y.w);
-    }
-    C[idx] = y;
+    float v[4] = {y[0], y[1], y[2], y[3]};
+    skinny_store(C, row, ocol, N, v, bias, flags);
 }
 
 // Mixed-dtype matmul: one thread per output, double accumulation in k order
@@ -2184,7 +2176,7 @@ using TileMid = Tile<128, 128, 32, 2, 2>;           // wave 64x64
 using TileMidK = Tile<128, 128, 64, 2, 2, 2, false>;
 using TileSmall = Tile<64, 64, 64, 2, 2, 2>;        // wave 32x32, two k-groups (8 waves)
 using TileTiny = Tile<32, 32, 64, 1, 1, 4>;         // one 32x32 block, four k-groups (4 waves)
-using TileSkinny = Tile<32, 128, 64, 1, 4>;  // M <= 32 when the streaming kernel cannot run
+using TileSkinny = Tile<32, 128, 64, 1, 4>;  // M <= 32 where the streaming kernel does not run (A transposed, N < 4)
 using TileConv = Tile<128, 128, 32, 2, 2>;   // NHWC conv, Co > 64, C % 32 == 0
 using TileConv16 = Tile<128, 128, 16, 2, 2>; // NHWC conv, Co > 64, C % 16 == 0
 using TileConv64 = Tile<64, 128, 32, 2, 2>;  // NHWC conv, Co <= 64, C % 32 == 0
@@ -2244,12 +2236,6 @@ int partial_buffer(size_t bytes, float **out) {
     return CAMEL_HIP_OK;
 }
 
-// True when the streaming skinny kernel serves C[M, N] = A[M, K] B[K, N].
-bool skinny_eligible(int64_t M, int64_t N, int64_t K, const float *B, const float *C) {
-    return M <= 32 && K > 0 && N % 4 == 0 && ((uintptr_t)B & 15) == 0 &&
-           ((uintptr_t)C & 15) == 0 && (K + SK_CHUNK - 1) / SK_CHUNK <= SK_MAX_KGROUPS;
-}
-
 // Shape of a skinny launch: chunks per work-group (ch) and work-groups along
 // K (nks; their partials need nks * M * N floats when nks > 1).
 struct SkinnyPlan {
@@ -2273,43 +2259,46 @@ SkinnyPlan plan_skinny(int64_t N, int64_t K) {
 
 size_t skinny_partial_bytes(int64_t M, int64_t N, int64_t K) {
     const SkinnyPlan p = plan_skinny(N, K);
-    return p.nks > 1 ? (size_t)p.nks * M * N * sizeof(float) : 0;
+    return p.nks > 1 ? (size_t)p.nks * M * ((N + 3) / 4 * 4) * sizeof(float) : 0;
+}
+
+// True when the streaming skinny kernel serves C[M, N] = A[M, K] B[K, N].  For
+// rows that are not 16-byte aligned it does while its partials fit the static
+// scratch: the tiles' K splits, at most 64, need less of it for the longest K.
+bool skinny_eligible(int64_t M, int64_t N, int64_t K, const float *B, const float *C) {
+    if (M > 32 || K <= 0 || N < 4 || (K + SK_CHUNK - 1) / SK_CHUNK > SK_MAX_KGROUPS) return false;
+    const bool aligned = N % 4 == 0 && ((uintptr_t)B & 15) == 0 && ((uintptr_t)C & 15) == 0;
+    return aligned || skinny_partial_bytes(M, N, K) <= CAMEL_HIP_NOALLOC_SCRATCH_BYTES;
 }
 
 int launch_skinny(const float *A, const float *B, float *C, int M, int N, int K, const float *bias,
                   int flags) {
     const int strips = (N + SK_COLS - 1) / SK_COLS;
-    const int ch = plan_skinny(N, K).ch;
-    const int mt = M <= 16 ? 1 : 2;
-    const int a_vec = M >= 16 * mt && K % 4 == 0 && ((uintptr_t)A & 15) == 0;
-    auto go = [&](auto kernel, int chunks) -> int {
-        const int nks = (K + SK_CHUNK * chunks - 1) / (SK_CHUNK * chunks);
+    const SkinnyPlan plan = plan_skinny(N, K);
+    const int mt = M <= 16 ? 1 : 2, ch = plan.ch, nks = plan.nks;
+    const size_t partial_bytes = skinny_partial_bytes(M, N, K);
+    auto go = [&](auto kernel) -> int {
         float *partial = nullptr;
-        if (nks > 1) CAMEL_RETURN_IF(partial_buffer((size_t)nks * M * N * sizeof(float), &partial));
+        if (nks > 1) CAMEL_RETURN_IF(partial_buffer(partial_bytes, &partial));
         hipLaunchKernelGGL(kernel, dim3((unsigned)strips, (unsigned)nks), dim3(SK_WAVES * 64), 0,
-                           stream(), A, B, C, M, N, K, bias, flags, partial, a_vec);
+                           stream(), A, B, C, M, N, K, bias, flags, partial);
         CAMEL_RETURN_IF(check_launch("sgemm_skinny_kernel"));
         if (nks == 1) return CAMEL_HIP_OK;
-        const int64_t total4 = (int64_t)M * N / 4;
-        const int by_strip = N % SK_COLS == 0 ? strips : 0;
-        const unsigned blocks =
-            by_strip ? (unsigned)(by_strip * ((M + 3) / 4))
-                     : (unsigned)((total4 + SK_REDUCE_THREADS - 1) / SK_REDUCE_THREADS);
-        hipLaunchKernelGGL(skinny_reduce_kernel, dim3(blocks), dim3(SK_REDUCE_THREADS), 0, stream(),
-                           reinterpret_cast<const float4 *>(partial), reinterpret_cast<float4 *>(C),
-                           M, N, nks, bias, flags, by_strip);
+        hipLaunchKernelGGL(skinny_reduce_kernel, dim3((unsigned)(strips * ((M + 3) / 4))),
+                           dim3(SK_REDUCE_THREADS), 0, stream(), reinterpret_cast<const float4 *>(partial),
+                           C, M, N, nks, bias, flags, strips);
         return check_launch("skinny_reduce_kernel");
     };
     if (mt == 1) {
-        if (ch == 8) return go(sgemm_skinny_kernel<1, 8>, 8);
-        if (ch == 4) return go(sgemm_skinny_kernel<1, 4>, 4);
-        if (ch == 2) return go(sgemm_skinny_kernel<1, 2>, 2);
-        return go(sgemm_skinny_kernel<1, 1>, 1);
+        if (ch == 8) return go(sgemm_skinny_kernel<1, 8>);
+        if (ch == 4) return go(sgemm_skinny_kernel<1, 4>);
+        if (ch == 2) return go(sgemm_skinny_kernel<1, 2>);
+        return go(sgemm_skinny_kernel<1, 1>);
     }
-    if (ch == 8) return go(sgemm_skinny_kernel<2, 8>, 8);
-    if (ch == 4) return go(sgemm_skinny_kernel<2, 4>, 4);
-    if (ch == 2) return go(sgemm_skinny_kernel<2, 2>, 2);
-    return go(sgemm_skinny_kernel<2, 1>, 1);
+    if (ch == 8) return go(sgemm_skinny_kernel<2, 8>);
+    if (ch == 4) return go(sgemm_skinny_kernel<2, 4>);
+    if (ch == 2) return go(sgemm_skinny_kernel<2, 2>);
+    return go(sgemm_skinny_kernel<2, 1>);
 }
 
 // Work-groups of one kernel that fit on the chip at once (occupancy x CUs).

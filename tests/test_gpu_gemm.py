@@ -288,3 +288,36 @@ def test_sgemm_special_values_propagate_like_the_reference(M, N, Kd):
     bound = 1e-5 * np.sqrt(Kd) * (np.abs(af) @ np.abs(bf))
     err = np.abs(got.astype(np.float64)[fin] - ref.astype(np.float64)[fin])
     assert np.all(err <= bound[fin] + 1e-30)
+
+
+@pytest.mark.parametrize("M,N,Kd", [
+    (1, 4, 1),         # one row, one column group, k below one MFMA
+    (5, 5, 3),         # the last group overlaps the first one
+    (16, 67, 128),     # group of 3 columns in the second strip, one whole chunk
+    (17, 63, 130),     # second 16-row group of one row, chunk of 2 k
+    (31, 1001, 777),   # rows of A and B at every alignment
+    (8, 4095, 4095),   # k groups whose partials have padded rows
+    (32, 2050, 8191),  # several chunks per work-group, ragged last one
+])
+def test_skinny_kernel_at_every_size_and_alignment(M, N, Kd):
+    # Operands whose sums are exact: equality to the bit.  Then an operand row
+    # and column of NaN, which may reach their own row and column only (rows
+    # and columns past the edge repeat the last ones).
+    from tests.test_gpu_exact import F, assert_bits, exact_dense, wide, wide_pair
+    print(f"skinny {M}x{N}x{Kd}", flush=True)
+    for side in ("A", "B"):
+        a, b = wide_pair(0x5300 + M + Kd, (M, Kd), (Kd, N), side)
+        bias = wide(0x5301 + N, (N,))
+        for skip in (0, 1):  # 4-byte aligned operands too
+            da, db = (K.dev(np.append(np.zeros(skip, F), v)) for v in (a, b))
+            dbias = K.dev(bias)
+            dc = K.empty(4 * (M * N + skip))
+            H.call("camel_hip_sgemm", K.P(da.ptr + 4 * skip), K.P(db.ptr + 4 * skip), K.P(dc.ptr + 4 * skip),
+                   M, N, Kd, K.P(dbias.ptr), H.EPI_BIAS | H.EPI_RELU)
+            got = K.host(dc, F, (M * N + skip,))[skip:].reshape(M, N)
+            assert_bits(got, exact_dense(a, b, bias, True), f"wide {side}, offset {skip}")
+    a[M - 1, Kd - 1] = b[Kd - 1, N - 1] = np.nan
+    got = K.sgemm(a, b, None, 0)
+    bad = np.zeros((M, N), bool)
+    bad[M - 1] = bad[:, N - 1] = True
+    assert np.array_equal(np.isnan(got), bad)
