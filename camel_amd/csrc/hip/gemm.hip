@@ -1663,7 +1663,7 @@ int launch_thin(const float *A, const float *B, float *C, int M, int N, int K, c
 // 16 on guarded loads 1 x 4096 x 4096 took 16.7 us, 14.4 without; 17 rows 21.7,
 // 17.4.  N % 4 != 0, on 32 x 128 tiles against here: 16 x 3001 x 2047 18.4 and
 // 12.1, 7 x 1001 x 77 7.7 and 4.0, 12 x 5 x 3000 16.9 and 6.7, 32 x 8191 x 8192
-// 78.5 and 69.6.)
+// 78.5 and 69.6.  16 aligned rows pay for the clamps: 16 x 4096 x 4096 14.70, 14.81.)
 constexpr int SK_WAVES = 8;
 constexpr int SK_COLS = 64;
 constexpr int SK_STEPS = 4;                          // 4-row MFMA steps per chunk and wave
