@@ -36,7 +36,8 @@ struct SplitConv {
     int pxs, cqs; // distance of pixels and (quads) of channel quads
     int shift;    // elements before x that the first window reaches back
     uint32_t bytes;          // of x and the shift before it
-    uint32_t mul_unit, mul_kw, mul_taps; // quotient_mul of unit, KW and taps
+    uint32_t mul_unit;                   // floor(k / unit) = k mul_unit >> 32
+    uint32_t mul_kw, mul_taps;           // tap_mul of KW and taps
     int patch, per_image;    // positions of a patch (0: not that kernel), tiles per image
     int w_packed;            // weights [Co][KH][KW][C], else [Co][C][KH][KW]
 };

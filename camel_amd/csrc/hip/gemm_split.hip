@@ -180,22 +180,21 @@ __device__ __forceinline__ void conv_k(const SplitConv &c, int k, int &tap, int 
     ch = blk * c.unit + k - run * c.unit;
 }
 
-// floor(n / d) for n, d < 65536 as one multiplication: the multiplier 2^32 / d
-// + 1, and 0 for d = 1, whose multiplier has 33 bits.
-constexpr uint32_t quotient_mul(uint32_t d) { return d == 1 ? 0 : (uint32_t)(((uint64_t)1 << 32) / d + 1); }
-__host__ __device__ __forceinline__ constexpr uint32_t quotient(uint32_t n, uint32_t mul) {
-    return mul ? (uint32_t)(((uint64_t)n * mul) >> 32) : n;
+// floor(n / d) for d <= 32 taps and n < 8192 runs of channels as a product: the
+// multiplier 2^18 / d + 1 fits 32 bits for d = 1 too, and the product as well.
+// (A branch for d = 1 in the stage loop: 16 x 96 x 55 x 55 stride 2 60 -> 68 us.)
+constexpr uint32_t tap_mul(uint32_t d) { return (1u << 18) / d + 1; }
+__host__ __device__ __forceinline__ constexpr uint32_t tap_quotient(uint32_t n, uint32_t mul) {
+    return n * mul >> 18;
 }
-constexpr bool quotients_hold() {
-    for (uint32_t d = 1; d <= 32; ++d)                    // taps by the kernel's width
-        for (uint32_t n = 0; n < 32; ++n)
-            if (quotient(n, quotient_mul(d)) != n / d) return false;
-    for (uint32_t d = 1; d <= 32; ++d)                    // runs by the taps: both ends of each quotient
-        for (uint32_t n = d; n < 8192; n += d)
-            if (quotient(n, quotient_mul(d)) != n / d || quotient(n - 1, quotient_mul(d)) != n / d - 1) return false;
+constexpr bool tap_quotients_hold() {
+    for (uint32_t d = 1; d <= 32; ++d)
+        for (uint32_t n = d; n <= 8192; n += d) // both ends of each quotient
+            if (tap_quotient(n - 1, tap_mul(d)) != n / d - 1 || (n < 8192 && tap_quotient(n, tap_mul(d)) != n / d))
+                return false;
     return true;
 }
-static_assert(quotients_hold(), "divisions of the convolution's k");
+static_assert(tap_quotients_hold(), "divisions of the convolution's k");
 
 // Element (k, n) of the im2col matrix.
 template <bool QUADS, bool POOL>
@@ -240,9 +239,9 @@ template <class T, bool QUADS, bool POOL> struct ConvB {
         taps[i] = m;
     }
     __device__ __forceinline__ void load(int i, int k, float *f) const {
-        const int run = (int)quotient(k, c.mul_unit), blk = (int)quotient(run, c.mul_taps);
+        const int run = (int)__umulhi((uint32_t)k, c.mul_unit), blk = (int)tap_quotient(run, c.mul_taps);
         const int tap = run - blk * c.taps, c0 = blk * c.unit + k - run * c.unit;
-        const int kh = (int)quotient(tap, c.mul_kw), kw = tap - kh * c.KW;
+        const int kh = (int)tap_quotient(tap, c.mul_kw), kw = tap - kh * c.KW;
         const uint32_t v = (taps[i] >> tap) & 1 ? off[i] : NO_ELEMENT;
         const uint32_t s = (uint32_t)((kh * c.W + kw) * c.pxs) * 4u;
         if constexpr (QUADS) {
@@ -1512,9 +1511,9 @@ int split_conv(SplitGemm g, SplitConv c, bool quads, bool pool, const SplitConvP
     c.per_image = plan.per_image;
     c.taps = c.KH * c.KW;
     c.unit = plan.blocked ? BK : (c.C + 7) / 8 * 8;
-    c.mul_unit = quotient_mul(c.unit);
-    c.mul_kw = quotient_mul(c.KW);
-    c.mul_taps = quotient_mul(c.taps);
+    c.mul_unit = (uint32_t)(((uint64_t)1 << 32) / c.unit + 1); // (unit >= 8, k < 65536)
+    c.mul_kw = tap_mul(c.KW);
+    c.mul_taps = tap_mul(c.taps);
     if (plan.blocked) g.K = (c.C + BK - 1) / BK * c.taps * BK;
     const int stages = (g.K + BK - 1) / BK;
     c.kpad = stages * BK - g.K;
