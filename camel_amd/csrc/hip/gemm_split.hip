@@ -1,10 +1,11 @@
 // fp32 GEMM on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16), which run 16
 // times the fp32 MFMA rate.
 //
-// Every fp32 operand x is taken as hi + mid + lo, three bf16 values: hi = x
-// rounded to nearest, mid = x - hi cut to 8 bits, lo = the rest.  24
-// significant bits make three 8-bit parts, so the sum is x exactly (|x| >=
-// 2^-100 and below the bf16 maximum; see below).  A product of two such
+// Every fp32 operand x is scaled by 2^24 and taken as hi + mid + lo, three bf16
+// values: hi = x rounded to nearest, mid = x - hi cut to 8 bits, lo = the rest.
+// 24 significant bits make three 8-bit parts, so the sum is x exactly: the last
+// bit of a scaled value is at least 2^-125, inside the bf16 range, for
+// subnormal x too.  The results are scaled back by 2^-48.  A product of two such
 // operands is the six part products down to 2^-18 of it -- hi hi, hi mid, mid
 // hi, mid mid, hi lo, lo hi -- each exact in fp32; the three dropped ones are
 // at most 2^-25 of the product, below the rounding of an fp32 product.
@@ -16,12 +17,11 @@
 // the fp32 MFMA chain, which rounds every 2 k.  (The 6 MFMAs on the
 // accumulator itself: 1.03e-6, 4% faster.)
 //
-// Operands outside the exact range, tile by tile: the converting lanes keep
-// the smallest nonzero |hi| (two packed 16-bit operations per pair), and a
-// value that is infinite, NaN or beyond the bf16 maximum makes its outputs
-// non-finite (its mid part is).  A tile that saw |x| < 2^-100 is computed again
-// in fp32 MFMA, and so are the non-finite sums of any other tile: special
-// values and the ends of the range give what they give in fp32.
+// The top of the range: |x| >= 2^104, infinities and NaN make hi infinite or NaN
+// and mid NaN, and a sum can pass 2^80 (the fp32 maximum, scaled).  Either way
+// the output is not finite, and a tile's non-finite outputs are formed again in
+// fp32 MFMA: special values and the ends of the range give what they give in
+// fp32.
 //
 // Tile: waves as WM x WN, each FM x FN blocks of 16 x 16; A goes from global
 // memory straight into the registers of the waves that multiply it (lane (r,
@@ -48,14 +48,12 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 
 constexpr int BK = 32;     // k per stage: one 16x16x32 MFMA
 constexpr int GROUP_M = 4; // tile rows per group of the XCD-aware order
 
-// 2 |hi| - 1 as 16-bit integers of a bf16 below 2^-100 (zero gives 0xffff).
-// From there on lo's last bit is at least 2^-123, inside the bf16 range.
-constexpr unsigned short TINY = (27 << 8) - 1;
+// The scale of each operand, and of the result back.
+constexpr float SCALE = 0x1p24f, UNSCALE = 0x1p-48f;
 
 // The upper halves of two floats, x0 in the lower half.
 __device__ __forceinline__ uint32_t upper_pair(float x0, float x1) {
@@ -65,30 +63,21 @@ __device__ __forceinline__ float upper(float x) {
     return __uint_as_float(__float_as_uint(x) & 0xffff0000u);
 }
 
-// tiny = min(tiny, 2 |h| - 1) over a pair of bf16.
-__device__ __forceinline__ void note_tiny(uint32_t h, us2 &tiny) {
-    us2 twice;
-    asm("v_pk_mad_u16 %0, %1, 2, -1 op_sel_hi:[1,0,0]" : "=v"(twice) : "v"(h));
-    tiny = __builtin_elementwise_min(tiny, twice);
-}
-
 // Pair c of f[0..7] (split8: all four) into three chunks of 8 bf16 (hi, mid,
-// lo); tiny: running minimum of 2 |hi| - 1.  (v_dot2_f32_bf16 with a -1 forms x - hi in one operation
-// instead of two, but its results may not be read for 3 wait states: 4096^3
-// 557 -> 578 us.)
-__device__ __forceinline__ void split_pair(const float *f, int c, u4 *out, us2 &tiny) {
-    float x0 = f[2 * c], x1 = f[2 * c + 1];
+// lo).  (v_dot2_f32_bf16 with a -1 forms x - hi in one operation instead of two,
+// but its results may not be read for 3 wait states: 4096^3 557 -> 578 us.)
+__device__ __forceinline__ void split_pair(const float *f, int c, u4 *out) {
+    float x0 = f[2 * c] * SCALE, x1 = f[2 * c + 1] * SCALE;
     const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){x0, x1}, bf2));
-    note_tiny(h, tiny);
     x0 = x0 - __uint_as_float(h << 16);
     x1 = x1 - __uint_as_float(h & 0xffff0000u);
     out[0][c] = h;
     out[1][c] = upper_pair(x0, x1);
     out[2][c] = upper_pair(x0 - upper(x0), x1 - upper(x1));
 }
-__device__ __forceinline__ void split8(const float *f, u4 *out, us2 &tiny) {
+__device__ __forceinline__ void split8(const float *f, u4 *out) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) split_pair(f, c, out, tiny);
+    for (int c = 0; c < 4; ++c) split_pair(f, c, out);
 }
 
 // WM x WN waves of FM x FN blocks; WK groups of them take alternate stages of
@@ -293,8 +282,7 @@ __global__ __launch_bounds__(64) void split_weights_kernel(SplitGemm g, SplitCon
 #pragma unroll
     for (int j = 0; j < 8; ++j) f[j] = k0 < 0 ? 0.f : conv_weight(g, c, row, k0 + j);
     u4 out[3];
-    us2 tiny = {0xffff, 0xffff};
-    split8(f, out, tiny);
+    split8(f, out);
     u4 *d = dst + ((size_t)stage * gridDim.y + blk) * 192 + lane;
 #pragma unroll
     for (int q = 0; q < 3; ++q) d[64 * q] = out[q];
@@ -407,13 +395,21 @@ __device__ __forceinline__ void store_conv(const SplitGemm &g, const SplitConv &
     }
 }
 
-// The sums of a tile that the split cannot form: all of them where an operand
-// was below its range (flag bit TINY_SEEN), the non-finite ones otherwise, in
-// fp32 (v_mfma_f32_16x16x4_f32, the same result layout), a few columns of
-// blocks at a time.  a(i, k), b(j, k): this lane's operand of block row i, column j.
-enum { TINY_SEEN = 1, NOT_FINITE = 2 };
+// Scales the sums back.
+template <int FM, int FN> __device__ __forceinline__ void unscale(f4 (*acc)[FN]) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[i][j][v] *= UNSCALE;
+}
+
+// The non-finite sums of a tile again in fp32 (v_mfma_f32_16x16x4_f32, the same
+// result layout), a few columns of blocks at a time.  a(i, k), b(j, k): this
+// lane's operand of block row i, column j.
 template <int FM, int FN, class A, class B>
-__device__ __forceinline__ void fp32_sums(f4 (*acc)[FN], int kbeg, int kend, bool all, int oct, A a, B b) {
+__device__ __forceinline__ void fp32_sums(f4 (*acc)[FN], int kbeg, int kend, int oct, A a, B b) {
     constexpr int JW = FN % 4 == 0 ? 4 : 2;
     static_assert(FN % JW == 0, "columns in groups");
     auto sums = [&](int j0, auto &y, int jy) {
@@ -449,7 +445,7 @@ __device__ __forceinline__ void fp32_sums(f4 (*acc)[FN], int kbeg, int kend, boo
                 for (int j = 0; j < JW; ++j)
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
-                        if (all || !(__builtin_fabsf(acc[i][j0 + j][v]) < INFINITY)) acc[i][j0 + j][v] = y[i][j][v];
+                        if (!(__builtin_fabsf(acc[i][j0 + j][v]) < INFINITY)) acc[i][j0 + j][v] = y[i][j][v];
         }
     }
 }
@@ -541,13 +537,12 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, 
             }
         }
     };
-    us2 tiny = {0xffff, 0xffff};
     auto store_patch = [&]() {
 #pragma unroll
         for (int i = 0; i < PATCH_IT; ++i) {
             if (64 * i >= c.patch) break;
             u4 d[3];
-            split8(raw[i], d, tiny);
+            split8(raw[i], d);
             if (64 * i + lane < PATCH)
 #pragma unroll
                 for (int q = 0; q < 3; ++q) patch[(q * 4 + wave) * PATCH + 64 * i + lane] = d[q];
@@ -599,12 +594,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, 
 #pragma unroll
             for (int i = 0; i < T::FM; ++i)
 #pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    a[i][q] = __builtin_bit_cast(bf8, an[i][q]);
-                    if (q == 0)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) note_tiny(an[i][0][e], tiny);
-                }
+                for (int q = 0; q < 3; ++q) a[i][q] = __builtin_bit_cast(bf8, an[i][q]);
             load_a(stage + 1);
             // next tap's offset (after the last one this tap's again)
             int next_off = tap_off + 1;
@@ -641,6 +631,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, 
         }
     }
 
+    unscale<T::FM, T::FN>(acc);
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < T::FM; ++i)
@@ -648,13 +639,12 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, 
         for (int j = 0; j < T::FN; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
-    if (bad) atomicOr(flag, (uint32_t)NOT_FINITE);
-    if (tiny.x < TINY || tiny.y < TINY) atomicOr(flag, (uint32_t)TINY_SEEN);
+    if (bad) *flag = 1;
     __syncthreads();
     const int mw = m0 + wm * T::FM * 16 + r16, nw = n0 + wn * T::FN * 16;
     if (*flag)
         fp32_sums<T::FM, T::FN>(
-            acc, 0, g.K, *flag & TINY_SEEN, oct,
+            acc, 0, g.K, oct,
             [&](int i, int k) { return conv_weight(g, c, min(mw + 16 * i, g.M - 1), k); },
             [&](int j, int k) { return conv_input<QUADS, POOL>(g, c, k, min(nw + 16 * j + r16, nend - 1)); });
     SplitGemm tile = g;
@@ -748,7 +738,6 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
             r < p.H ? reinterpret_cast<const f4 *>(xi)[tid] : f4{0.f, 0.f, 0.f, 0.f};
     }
     __syncthreads();
-    us2 tiny = {0xffff, 0xffff};
     const float *w1 = p.w1 + 8 * wave * 9;
 #pragma unroll 1
     for (int q = lane; q < PAIR_POS; q += 64) {
@@ -760,7 +749,7 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
         for (int e = 0; e < 8; ++e)
             f[e] = pair_conv1(xv, w1 + 9 * e, bias1 ? p.b1[8 * wave + e] : 0.f, bias1, relu1);
         u4 d[3];
-        split8(f, d, tiny);
+        split8(f, d);
 #pragma unroll
         for (int h = 0; h < 3; ++h) patch[(h * 4 + wave) * PAIR_POS + q] = d[h];
     }
@@ -793,12 +782,9 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
         for (int kw = 0; kw < 3; ++kw) {
             const int off = kh * PAIR_W + kw, next = kw < 2 ? off + 1 : min(kh + 1, 2) * PAIR_W;
 #pragma unroll
-            for (int i = 0; i < FM; ++i) {
+            for (int i = 0; i < FM; ++i)
 #pragma unroll
                 for (int q = 0; q < 3; ++q) a[i][q] = __builtin_bit_cast(bf8, an[i][q]);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) note_tiny(an[i][0][e], tiny);
-            }
             load_a(min(3 * kh + kw + 1, 8));
 #pragma unroll
             for (int j = 0; j < FN; ++j) {
@@ -828,6 +814,7 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
         }
     }
 
+    unscale<FM, FN>(acc);
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -835,8 +822,7 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
         for (int j = 0; j < FN; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
-    if (bad) atomicOr(&flag, (uint32_t)NOT_FINITE);
-    if (tiny.x < TINY || tiny.y < TINY) atomicOr(&flag, (uint32_t)TINY_SEEN);
+    if (bad) flag = 1;
     __syncthreads();
     if (flag) {
         SplitGemm g2{};
@@ -846,7 +832,7 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
         c2.taps = 9;
         c2.w_packed = p.w2_packed;
         fp32_sums<FM, FN>(
-            acc, 0, 9 * PAIR_C1, flag & TINY_SEEN, oct,
+            acc, 0, 9 * PAIR_C1, oct,
             [&](int i, int k) { return conv_weight(g2, c2, m0 + (wm * FM + i) * 16 + r16, k); },
             [&](int j, int k) {
                 const int col = (wn * FN + j) * 16 + r16, d = col & 3, tap = k / PAIR_C1, ch = k % PAIR_C1;
@@ -969,12 +955,11 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
 #pragma unroll
         for (int i = 0; i < T::B_IT; ++i) bsrc.load(i, k0 + 8 * b_oct[i], f[i]);
     };
-    us2 tiny = {0xffff, 0xffff};
     auto store_b = [&](u4 *lds, float (*f)[8]) {
 #pragma unroll
         for (int i = 0; i < T::B_IT; ++i) {
             u4 c[3];
-            split8(f[i], c, tiny);
+            split8(f[i], c);
 #pragma unroll
             for (int q = 0; q < 3; ++q) lds[q * 4 * T::BN + b_slot[i]] = c[q];
         }
@@ -987,10 +972,8 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
             if constexpr (ASRC == A_SPLIT) {
 #pragma unroll
                 for (int q = 0; q < 3; ++q) c[q] = r.c[i][q];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) note_tiny(c[0][q], tiny);
             } else {
-                split8(r.f[i], c, tiny);
+                split8(r.f[i], c);
             }
 #pragma unroll
             for (int q = 0; q < 3; ++q) a[i][q] = __builtin_bit_cast(bf8, c[q]);
@@ -1087,7 +1070,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
 #pragma unroll
             for (int u = 0; u < (SPREAD ? NB : 0); ++u) {
                 if (u * B_COLS / NB != j) continue;
-                split_pair(rb[u / 4], u % 4, cb, tiny);
+                split_pair(rb[u / 4], u % 4, cb);
                 if (u % 4 == 3) {
 #pragma unroll
                     for (int q = 0; q < 3; ++q) Bn[q * 4 * T::BN + b_slot[u / 4]] = cb[q];
@@ -1097,7 +1080,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
 #pragma unroll
             for (int u = 0; u < (SPREAD ? NA : 0); ++u) {
                 if (B_COLS + u * REST / (NA ? NA : 1) != j) continue;
-                split_pair(ra.f[u / 4], u % 4, an[u / 4], tiny);
+                split_pair(ra.f[u / 4], u % 4, an[u / 4]);
                 if (u % 4 == 3) load_a(k2, u / 4, ra);
             }
             if (j == T::FN - 2) __syncthreads();
@@ -1139,6 +1122,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
         add_t(T::FN - 1);
     }
 
+    unscale<T::FM, T::FN>(acc);
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < T::FM; ++i)
@@ -1146,8 +1130,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
         for (int j = 0; j < T::FN; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
-    if (bad) atomicOr(flag, (uint32_t)NOT_FINITE);
-    if (tiny.x < TINY || tiny.y < TINY) atomicOr(flag, (uint32_t)TINY_SEEN);
+    if (bad) *flag = 1;
     __syncthreads();
     if constexpr (T::WK > 1) {
         f4 *red = reinterpret_cast<f4 *>(smem);
@@ -1171,7 +1154,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
     const int nw = n0 + wn * T::FN * 16;
     if (*flag)
         fp32_sums<T::FM, T::FN>(
-            acc, max(ks0, 0), kend, *flag & TINY_SEEN, oct,
+            acc, max(ks0, 0), kend, oct,
             [&](int i, int k) {
                 const size_t m = min(mw + 16 * i, g.M - 1);
                 if constexpr (ASRC == A_SPLIT) return conv_weight(g, cv, (int)m, k);

@@ -108,6 +108,31 @@ def test_operands_outside_the_exact_range(M, N, Kd, trans):
     assert np.all(np.abs(got - ref) <= lim)
 
 
+@pytest.mark.parametrize("M,N,Kd,trans", SHAPES)
+def test_subnormal_operands_arrive(M, N, Kd, trans):
+    # One operand is a 1 (or 2^100) per column or row, the other one ordinary
+    # values with subnormal ones among them, down to the last bit of fp32: the
+    # product copies them, scaled.
+    print(f"split subnormal {M}x{N}x{Kd}", flush=True)
+    rng = np.random.default_rng(M + 5 * N)
+
+    def values(shape):
+        v = rng.uniform(-1, 1, shape).astype(F)
+        low = rng.random(shape) < 0.25
+        v[low] = (rng.uniform(-1, 1, low.sum()) * 2.0 ** rng.integers(-149, -133, low.sum())).astype(F)
+        return v
+
+    for factor in (F(1), F(2.0 ** 100)):
+        a, pick = values((M, Kd)), rng.integers(0, Kd, N)
+        b = np.zeros((Kd, N), F)
+        b[pick, np.arange(N)] = factor
+        assert_bits(run(a, b, None, 0, trans) + F(0), a[:, pick] * factor + F(0), f"A x {factor}")
+        b, pick = values((Kd, N)), rng.integers(0, Kd, M)
+        a = np.zeros((M, Kd), F)
+        a[np.arange(M), pick] = factor
+        assert_bits(run(a, b, None, 0, trans) + F(0), b[pick] * factor + F(0), f"B x {factor}")
+
+
 @pytest.mark.parametrize("M,N,Kd,trans", SHAPES[:4] + SHAPES[6:8])
 def test_special_values_propagate(M, N, Kd, trans):
     print(f"split special {M}x{N}x{Kd}", flush=True)
@@ -220,3 +245,54 @@ def test_conv_layouts_pool_and_special_values(geom):
     tiny = conv(x * F(2.0 ** -112), w, None, geom, 0).astype(np.float64) * 2.0 ** 112
     bound = 1e-5 * np.sqrt(C * KH * KW) * conv(np.abs(x), np.abs(w), None, geom, 0)
     assert np.all(np.abs(tiny - base) <= bound)
+
+
+@pytest.mark.parametrize("geom", CONVS)
+def test_conv_forms_agree_on_tiny_values(geom):
+    N, C, H_, W_, Co, KH, KW, st, pad = geom
+    # Inputs and weights with values far below the others, subnormal ones among
+    # them: every layout and the pooled form give the same bits, and a kernel
+    # that copies one tap of one channel copies subnormal inputs.
+    print(f"split conv tiny {geom}", flush=True)
+    rng = np.random.default_rng(C + 3 * Co)
+    x = rng.uniform(-1, 1, (N, C, H_, W_)).astype(F)
+    w = rng.uniform(-1, 1, (Co, C, KH, KW)).astype(F)
+    for arr in (x, w):
+        v = arr.reshape(-1)
+        at = rng.choice(v.size, size=max(1, v.size // 3000), replace=False)
+        v[at] = (rng.uniform(-1, 1, at.size) * 2.0 ** rng.integers(-149, -90, at.size)).astype(F)
+    y = conv(x, w, None, geom, 0)
+    if C % 4 == 0:
+        for layout in (H.CONV_X_NHWC, H.CONV_X_NCHW4):
+            np.testing.assert_array_equal(conv(x, w, None, geom, 0, layout=layout), y)
+    if min(y.shape[2:]) >= 2:
+        np.testing.assert_array_equal(conv(x, w, None, geom, 0, pool=True), pooled(y))
+    xs = (rng.uniform(-1, 1, x.shape) * 2.0 ** -138).astype(F)
+    ws = np.zeros_like(w)
+    ws[:, 0, 0, 0] = 1.0
+    got = conv(xs, ws, None, geom, 0)
+    OH, OW = got.shape[2:]
+    xp = np.zeros((N, H_ + 2 * pad, W_ + 2 * pad), F)
+    xp[:, pad:pad + H_, pad:pad + W_] = xs[:, 0]
+    want = xp[:, 0:st * (OH - 1) + 1:st, 0:st * (OW - 1) + 1:st]
+    np.testing.assert_array_equal(got, np.broadcast_to(want[:, None], got.shape))
+
+
+@pytest.mark.parametrize("tiny", ["x", "w2", "one pixel"])
+def test_conv_pair_equals_its_calls_on_tiny_values(tiny):
+    from tests.test_gpu_fusion import _pair_fused, _pair_unfused
+    print(f"split pair tiny {tiny}", flush=True)
+    rng = np.random.default_rng(0x5400)
+    x = rng.uniform(-1, 1, (3, 1, 28, 28)).astype(F)
+    w1 = rng.uniform(-1, 1, (32, 1, 3, 3)).astype(F)
+    w2 = rng.uniform(-1, 1, (64, 32, 3, 3)).astype(F)
+    if tiny == "x":
+        x[:, :, 4:12, 5:14] *= F(2.0 ** -120)
+    elif tiny == "w2":
+        w2[3, 5, 1, 1], w2[40, 7, 0, 2] = 1e-40, 1e-33
+    else:
+        x[...] = 0
+        x[1, 0, 14, 14] = 1e-38
+    want = _pair_unfused(x, w1, None, w2, None, 0, 0)
+    assert want.any()
+    np.testing.assert_array_equal(_pair_fused(x, w1, None, w2, None, 0, 0), want)
