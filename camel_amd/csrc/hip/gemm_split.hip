@@ -19,9 +19,9 @@
 //
 // The top of the range: |x| >= 2^104, infinities and NaN make hi infinite or NaN
 // and mid NaN, and a sum can pass 2^80 (the fp32 maximum, scaled).  Either way
-// the output is not finite, and a tile's non-finite outputs are formed again in
-// fp32 MFMA: special values and the ends of the range give what they give in
-// fp32.
+// the output is not finite, and non-finite outputs, each by itself, are formed
+// again in fp32 MFMA: special values and the ends of the range give what they
+// give in fp32, and no output depends on another row or column.
 //
 // Tile: waves as WM x WN, each FM x FN blocks of 16 x 16; A goes from global
 // memory straight into the registers of the waves that multiply it (lane (r,
@@ -395,58 +395,64 @@ __device__ __forceinline__ void store_conv(const SplitGemm &g, const SplitConv &
     }
 }
 
-// Scales the sums back.
-template <int FM, int FN> __device__ __forceinline__ void unscale(f4 (*acc)[FN]) {
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[i][j][v] *= UNSCALE;
-}
-
-// The non-finite sums of a tile again in fp32 (v_mfma_f32_16x16x4_f32, the same
-// result layout), a few columns of blocks at a time.  a(i, k), b(j, k): this
-// lane's operand of block row i, column j.
-template <int FM, int FN, class A, class B>
-__device__ __forceinline__ void fp32_sums(f4 (*acc)[FN], int kbeg, int kend, int oct, A a, B b) {
-    constexpr int JW = FN % 4 == 0 ? 4 : 2;
+// Scales a wave's sums back and forms its non-finite ones, and no others, again
+// in fp32 (v_mfma_f32_16x16x4_f32, the same result layout): JW columns of blocks
+// at a time, where any of them holds one.  a(i, k), b(j, k): this lane's
+// operand of block row i, column j; a lane's k of 32 are 8 consecutive ones,
+// loaded together.
+template <int FM, int FN, int JW, int S, class A, class B>
+__device__ __forceinline__ void finish_sums(f4 (*acc)[FN], int kbeg, int kend, int oct, A a, B b) {
     static_assert(FN % JW == 0, "columns in groups");
-    auto sums = [&](int j0, auto &y, int jy) {
+#pragma unroll
+    for (int j0 = 0; j0 < FN; j0 += JW) {
+        bool bad = false;
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < JW; ++j) y[i][jy + j] = f4{0.f, 0.f, 0.f, 0.f};
+            for (int j = j0; j < j0 + JW; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    acc[i][j][v] *= UNSCALE;
+                    bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
+                }
+        if (!__any(bad)) continue;
+        f4 y[FM][JW];
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < JW; ++j) y[i][j] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-        for (int k0 = kbeg; k0 < kend; k0 += 4) {
-            const int k = k0 + oct;
-            float fa[FM], fb[JW];
+        for (int k0 = kbeg; k0 < kend; k0 += 4 * S) {
+            float fa[FM][S], fb[JW][S];
 #pragma unroll
-            for (int i = 0; i < FM; ++i) fa[i] = k < kend ? a(i, k) : 0.f;
+            for (int s = 0; s < S; ++s) {
+                const int k = min(k0 + S * oct + s, kend - 1);
 #pragma unroll
-            for (int j = 0; j < JW; ++j) fb[j] = k < kend ? b(j0 + j, k) : 0.f;
+                for (int i = 0; i < FM; ++i) fa[i][s] = a(i, k);
 #pragma unroll
-            for (int i = 0; i < FM; ++i)
+                for (int j = 0; j < JW; ++j) fb[j][s] = b(j0 + j, k);
+            }
 #pragma unroll
-                for (int j = 0; j < JW; ++j)
-                    y[i][jy + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j], fa[i], y[i][jy + j], 0, 0, 0);
+            for (int s = 0; s < S; ++s) {
+                const bool in = k0 + S * oct + s < kend; // past the end both are zero
+#pragma unroll
+                for (int j = 0; j < JW; ++j) fb[j][s] = in ? fb[j][s] : 0.f;
+#pragma unroll
+                for (int i = 0; i < FM; ++i) {
+                    fa[i][s] = in ? fa[i][s] : 0.f;
+#pragma unroll
+                    for (int j = 0; j < JW; ++j)
+                        y[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j][s], fa[i][s], y[i][j], 0, 0, 0);
+                }
+            }
         }
-    };
 #pragma unroll
-    for (int j0 = 0; j0 < FN; j0 += JW) {
-        if constexpr (FM * FN > 16) { // no registers for both: all of them
-            sums(j0, acc, j0);
-        } else {
-            f4 y[FM][JW];
-            sums(j0, y, 0);
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int i = 0; i < FM; ++i)
+            for (int j = 0; j < JW; ++j)
 #pragma unroll
-                for (int j = 0; j < JW; ++j)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        if (!(__builtin_fabsf(acc[i][j0 + j][v]) < INFINITY)) acc[i][j0 + j][v] = y[i][j][v];
-        }
+                for (int v = 0; v < 4; ++v)
+                    if (!(__builtin_fabsf(acc[i][j0 + j][v]) < INFINITY)) acc[i][j0 + j][v] = y[i][j][v];
     }
 }
 
@@ -473,8 +479,7 @@ constexpr int PATCH_IT = (PATCH + 63) / 64;
 
 template <class T, bool QUADS, bool POOL>
 __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, SplitConv c) {
-    __shared__ u4 patch[12 * PATCH + 1];
-    uint32_t *const flag = reinterpret_cast<uint32_t *>(patch + 12 * PATCH);
+    __shared__ u4 patch[12 * PATCH];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / T::WN, wn = wave - wm * T::WN;
@@ -490,7 +495,6 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, 
     const int n0 = c.per_image ? tn / tiles_i * per + tn % tiles_i * T::BN : tn * T::BN;
     const int nend = c.per_image ? (tn / tiles_i + 1) * per : g.N;
     const int Hp = c.H + 2 * c.pad, Wp = c.W + 2 * c.pad, taps = c.taps;
-    if (tid == 0) *flag = 0;
     auto position = [&](int n) {
         int img, oh, ow;
         conv_pixel<POOL>(c, min(n, nend - 1), img, oh, ow);
@@ -631,22 +635,10 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, 
         }
     }
 
-    unscale<T::FM, T::FN>(acc);
-    bool bad = false;
-#pragma unroll
-    for (int i = 0; i < T::FM; ++i)
-#pragma unroll
-        for (int j = 0; j < T::FN; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
-    if (bad) *flag = 1;
-    __syncthreads();
     const int mw = m0 + wm * T::FM * 16 + r16, nw = n0 + wn * T::FN * 16;
-    if (*flag)
-        fp32_sums<T::FM, T::FN>(
-            acc, 0, g.K, oct,
-            [&](int i, int k) { return conv_weight(g, c, min(mw + 16 * i, g.M - 1), k); },
-            [&](int j, int k) { return conv_input<QUADS, POOL>(g, c, k, min(nw + 16 * j + r16, nend - 1)); });
+    finish_sums<T::FM, T::FN, 4, 2>(
+        acc, 0, g.K, oct, [&](int i, int k) { return conv_weight(g, c, min(mw + 16 * i, g.M - 1), k); },
+        [&](int j, int k) { return conv_input<QUADS, POOL>(g, c, k, min(nw + 16 * j + r16, nend - 1)); });
     SplitGemm tile = g;
     tile.N = nend;
     tile.partial = nullptr;
@@ -708,7 +700,6 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
     constexpr int FM = 2, FN = PAIR_FN;
     __shared__ u4 patch[12 * PAIR_POS];
     __shared__ __attribute__((aligned(16))) float img[PAIR_IR * PAIR_W];
-    __shared__ uint32_t flag;
     const bool bias1 = p.flags1 & CAMEL_EPI_BIAS, relu1 = p.flags1 & CAMEL_EPI_RELU;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -729,7 +720,6 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
             for (int q = 0; q < 3; ++q) an[i][q] = a_src[i][(size_t)tap * a_blocks * 192 + 64 * q];
     };
     load_a(0);
-    if (tid == 0) flag = 0;
     // The band's input rows, 16 bytes per thread (zeros past the image: never
     // read by a valid output).
     if (tid < PAIR_IR * PAIR_W / 4) {
@@ -814,36 +804,24 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
         }
     }
 
-    unscale<FM, FN>(acc);
-    bool bad = false;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
-    if (bad) flag = 1;
-    __syncthreads();
-    if (flag) {
-        SplitGemm g2{};
-        SplitConv c2{};
-        g2.A = p.w2;
-        c2.C = c2.unit = PAIR_C1;
-        c2.taps = 9;
-        c2.w_packed = p.w2_packed;
-        fp32_sums<FM, FN>(
-            acc, 0, 9 * PAIR_C1, oct,
-            [&](int i, int k) { return conv_weight(g2, c2, m0 + (wm * FM + i) * 16 + r16, k); },
-            [&](int j, int k) {
-                const int col = (wn * FN + j) * 16 + r16, d = col & 3, tap = k / PAIR_C1, ch = k % PAIR_C1;
-                int py, px;
-                pair_window(col, py, px);
-                const int r = 2 * py + (d >> 1) + tap / 3, c = 2 * px + (d & 1) + tap % 3;
-                float xv[9];
-                for (int e = 0; e < 9; ++e) xv[e] = img[(r + e / 3) * PAIR_W + c + e % 3];
-                return pair_conv1(xv, p.w1 + 9 * ch, bias1 ? p.b1[ch] : 0.f, bias1, relu1);
-            });
-    }
+    SplitGemm g2{};
+    SplitConv c2{};
+    g2.A = p.w2;
+    c2.C = c2.unit = PAIR_C1;
+    c2.taps = 9;
+    c2.w_packed = p.w2_packed;
+    finish_sums<FM, FN, 2, 2>(
+        acc, 0, 9 * PAIR_C1, oct,
+        [&](int i, int k) { return conv_weight(g2, c2, m0 + (wm * FM + i) * 16 + r16, k); },
+        [&](int j, int k) {
+            const int col = (wn * FN + j) * 16 + r16, d = col & 3, tap = k / PAIR_C1, ch = k % PAIR_C1;
+            int py, px;
+            pair_window(col, py, px);
+            const int r = 2 * py + (d >> 1) + tap / 3, c = 2 * px + (d & 1) + tap % 3;
+            float xv[9];
+            for (int e = 0; e < 9; ++e) xv[e] = img[(r + e / 3) * PAIR_W + c + e % 3];
+            return pair_conv1(xv, p.w1 + 9 * ch, bias1 ? p.b1[ch] : 0.f, bias1, relu1);
+        });
     // bias, relu, then the window's maximum: first, then strict '>'
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
@@ -873,8 +851,7 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
 template <class T, int ASRC, class BSrc, int OUT>
 __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, SplitConv cv) {
     constexpr bool AT = ASRC == A_COLS;
-    __shared__ u4 smem[T::LDS + 1];
-    uint32_t *const flag = reinterpret_cast<uint32_t *>(smem + T::LDS);
+    __shared__ u4 smem[T::LDS];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kg = T::WK > 1 ? wave / T::GW : 0, w = wave - kg * T::GW;
@@ -896,7 +873,6 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
     const int ns = (kend - ks0) / T::SB;
     const int kbeg = ks0 + kg * BK;
     u4 *const bufs = smem + kg * 2 * T::B_ST;
-    if (tid == 0) *flag = 0;
 
     // Rows and columns past the problem repeat the last one (never stored).
     const int mw = m0 + wm * T::FM * 16 + r16;
@@ -1122,17 +1098,8 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
         add_t(T::FN - 1);
     }
 
-    unscale<T::FM, T::FN>(acc);
-    bool bad = false;
-#pragma unroll
-    for (int i = 0; i < T::FM; ++i)
-#pragma unroll
-        for (int j = 0; j < T::FN; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
-    if (bad) *flag = 1;
-    __syncthreads();
     if constexpr (T::WK > 1) {
+        __syncthreads(); // the last operand reads
         f4 *red = reinterpret_cast<f4 *>(smem);
         if (kg > 0) {
 #pragma unroll
@@ -1152,15 +1119,14 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
                     acc[i][j] += red[((q * T::GW + w) * T::FM * T::FN + i * T::FN + j) * 64 + lane];
     }
     const int nw = n0 + wn * T::FN * 16;
-    if (*flag)
-        fp32_sums<T::FM, T::FN>(
-            acc, max(ks0, 0), kend, oct,
-            [&](int i, int k) {
-                const size_t m = min(mw + 16 * i, g.M - 1);
-                if constexpr (ASRC == A_SPLIT) return conv_weight(g, cv, (int)m, k);
-                return AT ? g.A[(size_t)k * g.lda + m] : g.A[m * g.lda + k];
-            },
-            [&](int j, int k) { return BSrc::at(g, cv, k, min(nw + 16 * j + r16, g.N - 1)); });
+    finish_sums<T::FM, T::FN, 4, (ASRC == A_SPLIT ? 2 : T::FM * T::FN > 16 ? 4 : 8)>(
+        acc, max(ks0, 0), kend, oct,
+        [&](int i, int k) {
+            const size_t m = min(mw + 16 * i, g.M - 1);
+            if constexpr (ASRC == A_SPLIT) return conv_weight(g, cv, (int)m, k);
+            return AT ? g.A[(size_t)k * g.lda + m] : g.A[m * g.lda + k];
+        },
+        [&](int j, int k) { return BSrc::at(g, cv, k, min(nw + 16 * j + r16, g.N - 1)); });
     if constexpr (OUT == OUT_MATRIX)
         store_matrix<T::FM, T::FN>(g, acc, split, mw, nw + 4 * oct);
     else

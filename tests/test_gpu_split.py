@@ -133,6 +133,40 @@ def test_subnormal_operands_arrive(M, N, Kd, trans):
         assert_bits(run(a, b, None, 0, trans) + F(0), b[pick] * factor + F(0), f"B x {factor}")
 
 
+@pytest.mark.parametrize("M,N,Kd,trans", SHAPES)
+def test_outputs_depend_on_their_own_row_and_column(M, N, Kd, trans):
+    # A special value in one row of A and one column of B changes no bit
+    # elsewhere.
+    print(f"split own {M}x{N}x{Kd}", flush=True)
+    rng = np.random.default_rng(M + 11 * N)
+    a = rng.uniform(-1, 1, (M, Kd)).astype(F)
+    b = rng.uniform(-1, 1, (Kd, N)).astype(F)
+    base = run(a, b, None, 0, trans)
+    rest = np.ix_(np.arange(M) != 1, np.arange(N) != N - 2)
+    for value in (1e-33, 1e-42, 1e32, np.finfo(F).max, np.inf, np.nan):
+        a2, b2 = a.copy(), b.copy()
+        a2[1, Kd - 1] = b2[0, N - 2] = value
+        assert_bits(run(a2, b2, None, 0, trans)[rest], base[rest], f"{value}")
+
+
+@pytest.mark.parametrize("M,N,Kd,trans", SHAPES)
+def test_sums_beyond_the_scaled_range(M, N, Kd, trans):
+    # Sums past 2^80, the fp32 maximum once scaled, are formed in fp32, to the
+    # fp32 kernels' bound; those below stay as they are.
+    print(f"split large {M}x{N}x{Kd}", flush=True)
+    rng = np.random.default_rng(M + 17 * Kd)
+    a = rng.uniform(-1, 1, (M, Kd)).astype(F)
+    b = rng.uniform(-1, 1, (Kd, N)).astype(F)
+    base = run(a, b, None, 0, trans)
+    big = np.arange(M) % 3 == 0
+    a[big] *= F(2.0 ** 50)
+    got = run(a, b * F(2.0 ** 45), None, 0, trans)
+    assert_bits(got[~big], base[~big] * F(2.0 ** 45), "small rows")
+    a64, b64 = a.astype(np.float64), b.astype(np.float64) * 2.0 ** 45
+    bound = 1e-5 * np.sqrt(Kd) * (np.abs(a64[big]) @ np.abs(b64))
+    assert np.all(np.abs(got[big] - a64[big] @ b64) <= bound)
+
+
 @pytest.mark.parametrize("M,N,Kd,trans", SHAPES[:4] + SHAPES[6:8])
 def test_special_values_propagate(M, N, Kd, trans):
     print(f"split special {M}x{N}x{Kd}", flush=True)
