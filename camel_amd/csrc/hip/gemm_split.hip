@@ -2,13 +2,13 @@
 // times the fp32 MFMA rate.
 //
 // Every fp32 operand x is scaled by 2^24 and taken as hi + mid + lo, three bf16
-// values: hi = x rounded to nearest, mid = x - hi cut to 8 bits, lo = the rest.
+// values: hi = x and mid = x - hi rounded to nearest, lo = the rest.
 // 24 significant bits make three 8-bit parts, so the sum is x exactly: the last
 // bit of a scaled value is at least 2^-125, inside the bf16 range, for
 // subnormal x too.  The results are scaled back by 2^-48.  A product of two such
-// operands is the six part products down to 2^-18 of it -- hi hi, hi mid, mid
-// hi, mid mid, hi lo, lo hi -- each exact in fp32; the three dropped ones are
-// at most 2^-25 of the product, below the rounding of an fp32 product.
+// operands is the six part products hi hi, hi mid, mid hi, mid mid, hi lo, lo
+// hi, each exact in fp32.  The three others are dropped: |mid| <= 2^-8 and |lo| <=
+// 2^-17 of the leading bit, so they are at most 2^-24 (1 + 2^-9) of the product.
 //
 // Sums: the 6 MFMAs of a 16 x 16 block and 32 k start from zero, smallest
 // products first, and their sum is added to the block's fp32 accumulator on
@@ -17,11 +17,23 @@
 // the fp32 MFMA chain, which rounds every 2 k.  (The 6 MFMAs on the
 // accumulator itself: 1.03e-6, 4% faster.)
 //
+// One product by itself: the MFMA cuts its sum where an fp32 product rounds, so
+// a sum of one term is off by up to 1.5 units of its last place (the cut 1, the
+// dropped products 0.5; measured 1.46, 2-norm 3.1e-8 against 2.5e-8 of a rounded
+// product).  With hi hi in a sum of its own, added on the vector ALU, it is 1.0
+// (measured 0.96, 2-norm 2.5e-8); the 64 x 64 tile, whose three chains need that
+// add anyway, does so, the others would run 3 to 7% longer (4096^3 537 -> 567 us,
+// conv 64 x 64 x 56 x 56 140 -> 150).  With the two products mid lo and lo mid as
+// well it is 0.51 (measured), at 4096^3 537 -> 685.  Sums of more terms are
+// more exact than the fp32 chain's in all forms: 64 terms 4.5e-8 against 1.4e-7.
+//
 // The top of the range: |x| >= 2^104, infinities and NaN make hi infinite or NaN
 // and mid NaN, and a sum can pass 2^80 (the fp32 maximum, scaled).  Either way
 // the output is not finite, and non-finite outputs, each by itself, are formed
 // again in fp32 MFMA: special values and the ends of the range give what they
 // give in fp32, and no output depends on another row or column.
+// That takes time only where such values are: 4096^3 550 us (fp32 kernels 960),
+// with one infinity 1560, with all sums past 2^80 2510.
 //
 // Tile: waves as WM x WN, each FM x FN blocks of 16 x 16; A goes from global
 // memory straight into the registers of the waves that multiply it (lane (r,
@@ -59,25 +71,38 @@ constexpr float SCALE = 0x1p24f, UNSCALE = 0x1p-48f;
 __device__ __forceinline__ uint32_t upper_pair(float x0, float x1) {
     return __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
 }
-__device__ __forceinline__ float upper(float x) {
-    return __uint_as_float(__float_as_uint(x) & 0xffff0000u);
-}
 
 // Pair c of f[0..7] (split8: all four) into three chunks of 8 bf16 (hi, mid,
 // lo).  (v_dot2_f32_bf16 with a -1 forms x - hi in one operation instead of two,
 // but its results may not be read for 3 wait states: 4096^3 557 -> 578 us.)
 __device__ __forceinline__ void split_pair(const float *f, int c, u4 *out) {
-    float x0 = f[2 * c] * SCALE, x1 = f[2 * c + 1] * SCALE;
+    // (The factor in a scalar register instead of a literal: half the size of the
+    // multiplication; 16 x 96 x 55 x 55 stride 2 60.8 -> 56.7 us.)
+    float scale = SCALE;
+    asm("" : "+s"(scale));
+    float x0 = f[2 * c] * scale, x1 = f[2 * c + 1] * scale;
     const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){x0, x1}, bf2));
     x0 = x0 - __uint_as_float(h << 16);
     x1 = x1 - __uint_as_float(h & 0xffff0000u);
+    const uint32_t m = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){x0, x1}, bf2));
     out[0][c] = h;
-    out[1][c] = upper_pair(x0, x1);
-    out[2][c] = upper_pair(x0 - upper(x0), x1 - upper(x1));
+    out[1][c] = m;
+    out[2][c] = upper_pair(x0 - __uint_as_float(m << 16), x1 - __uint_as_float(m & 0xffff0000u));
 }
 __device__ __forceinline__ void split8(const float *f, u4 *out) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) split_pair(f, c, out);
+}
+
+// Operands of the part products, smallest first: (lo hi), (hi lo), (mid mid),
+// (mid hi), (hi mid), (hi hi).
+constexpr int PRODUCTS = 6;
+constexpr int PA[PRODUCTS] = {2, 0, 1, 1, 0, 0}, PB[PRODUCTS] = {0, 2, 1, 0, 1, 0};
+
+// Adds the scaled products of 32 k to a block's accumulator.
+__device__ __forceinline__ void add_products(f4 &acc, f4 t) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[v] = __builtin_fmaf(t[v], UNSCALE, acc[v]);
 }
 
 // WM x WN waves of FM x FN blocks; WK groups of them take alternate stages of
@@ -395,7 +420,7 @@ __device__ __forceinline__ void store_conv(const SplitGemm &g, const SplitConv &
     }
 }
 
-// Scales a wave's sums back and forms its non-finite ones, and no others, again
+// Forms a wave's non-finite sums, and no others, again
 // in fp32 (v_mfma_f32_16x16x4_f32, the same result layout): JW columns of blocks
 // at a time, where any of them holds one.  a(i, k), b(j, k): this lane's
 // operand of block row i, column j; a lane's k of 32 are 8 consecutive ones,
@@ -411,10 +436,7 @@ __device__ __forceinline__ void finish_sums(f4 (*acc)[FN], int kbeg, int kend, i
 #pragma unroll
             for (int j = j0; j < j0 + JW; ++j)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    acc[i][j][v] *= UNSCALE;
-                    bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
-                }
+                for (int v = 0; v < 4; ++v) bad |= !(__builtin_fabsf(acc[i][j][v]) < INFINITY);
         if (!__any(bad)) continue;
         f4 y[FM][JW];
 #pragma unroll
@@ -585,7 +607,6 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, 
         for (int q = 0; q < 3; ++q)
             d[q] = __builtin_bit_cast(bf8, patch[q * 4 * PATCH + at[j] + tap_off]);
     };
-    constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
     int stage = 0;
     for (int blk = 0; blk < blocks; ++blk) {
         if (blk > 0) __syncthreads(); // the block before is multiplied
@@ -613,16 +634,16 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, 
 #pragma unroll
                 for (int i = 0; i < T::FM; ++i) t[j & 1][i] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int p = 0; p < 6; ++p)
+                for (int p = 0; p < PRODUCTS; ++p)
 #pragma unroll
                     for (int i = 0; i < T::FM; ++i)
                         t[j & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j & 1][PB[p]], a[i][PA[p]],
                                                                               t[j & 1][i], 0, 0, 0);
 #pragma unroll
                 for (int i = 0; i < T::FM; ++i)
-                    if (j > 0) acc[i][j - 1] += t[(j + 1) & 1][i];
+                    if (j > 0) add_products(acc[i][j - 1], t[(j + 1) & 1][i]);
 #pragma unroll
-                for (int r = 0; r < 6 * T::FM; ++r) {
+                for (int r = 0; r < PRODUCTS * T::FM; ++r) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                     if (r % T::FM == T::FM - 1 && r < 3 * T::FM) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                     if (r >= T::FM) __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
@@ -630,7 +651,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, 
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int i = 0; i < T::FM; ++i) acc[i][T::FN - 1] += t[(T::FN - 1) & 1][i];
+            for (int i = 0; i < T::FM; ++i) add_products(acc[i][T::FN - 1], t[(T::FN - 1) & 1][i]);
             tap_off = next_off;
         }
     }
@@ -765,7 +786,6 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
         for (int q = 0; q < 3; ++q) d[q] = __builtin_bit_cast(bf8, patch[q * 4 * PAIR_POS + at[j] + off]);
     };
     fetch(0, 0, b[0]);
-    constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll 1
     for (int kh = 0; kh < 3; ++kh) {
 #pragma unroll
@@ -783,16 +803,16 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
 #pragma unroll
                 for (int i = 0; i < FM; ++i) t[u][i] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int q = 0; q < 6; ++q)
+                for (int q = 0; q < PRODUCTS; ++q)
 #pragma unroll
                     for (int i = 0; i < FM; ++i)
                         t[u][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[u][PB[q]], a[i][PA[q]], t[u][i], 0,
                                                                           0, 0);
                 if (j > 0)
 #pragma unroll
-                    for (int i = 0; i < FM; ++i) acc[i][j - 1] += t[u ^ 1][i];
+                    for (int i = 0; i < FM; ++i) add_products(acc[i][j - 1], t[u ^ 1][i]);
 #pragma unroll
-                for (int r = 0; r < 6 * FM; ++r) {
+                for (int r = 0; r < PRODUCTS * FM; ++r) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                     if (r % FM == FM - 1 && r < 3 * FM) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                     if (r >= FM) __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
@@ -800,7 +820,7 @@ __global__ __launch_bounds__(256, 2) void conv_pair_kernel(SplitPair p, const u4
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int i = 0; i < FM; ++i) acc[i][FN - 1] += t[(kw * FN + FN - 1) & 1][i];
+            for (int i = 0; i < FM; ++i) add_products(acc[i][FN - 1], t[(kw * FN + FN - 1) & 1][i]);
         }
     }
 
@@ -989,14 +1009,17 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
     __syncthreads();
     const int b_rd = oct * T::BN + wn * T::FN * 16 + r16;
     bf8 b[2][3];
-    // A wave of one block row runs its six products as two chains, so that no
-    // MFMA waits for the one before.
-    constexpr int NC = T::FM == 1 ? 2 : 1;
+    // A wave of one block row runs its six products as three chains, so that no
+    // MFMA waits for the one before; hi hi is one of its own, which the vector
+    // ALU adds rounded.
+    constexpr int NC = T::FM == 1 ? 3 : 1;
     f4 t[2][T::FM * NC];
     auto add_t = [&](int j) {
+        if constexpr (NC == 3)
+            add_products(acc[0][j], (t[j & 1][0] + t[j & 1][1]) + t[j & 1][2]);
+        else
 #pragma unroll
-        for (int i = 0; i < T::FM; ++i)
-            acc[i][j] += NC == 2 ? t[j & 1][i] + t[j & 1][i + NC - 1] : t[j & 1][i];
+            for (int i = 0; i < T::FM; ++i) add_products(acc[i][j], t[j & 1][i]);
     };
     auto fetch = [&](const u4 *Bs, int j, bf8 *d) {
 #pragma unroll
@@ -1004,9 +1027,6 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
             d[q] = __builtin_bit_cast(bf8, Bs[q * 4 * T::BN + b_rd + 16 * j]);
     };
     fetch(bufs, 0, b[0]);
-    // part products, smallest first: (lo hi), (hi lo), (mid mid), (mid hi),
-    // (hi mid), (hi hi)
-    constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
     // SPREAD: the conversions of the next stage, a pair of values at a time,
     // over the columns, so that they run in the shadow of the MFMAs: B's pairs
     // in the first half (before the barrier column), A's in the second, each
@@ -1032,10 +1052,10 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
 #pragma unroll
             for (int i = 0; i < T::FM * NC; ++i) t[j & 1][i] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int p = 0; p < 6; ++p)
+            for (int p = 0; p < PRODUCTS; ++p)
 #pragma unroll
                 for (int i = 0; i < T::FM; ++i) {
-                    f4 &c = t[j & 1][i + p % NC];
+                    f4 &c = t[j & 1][i + (NC == 1 ? 0 : p + 1 < PRODUCTS ? p % 2 : 2)];
                     c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j & 1][PB[p]], a[i][PA[p]], c, 0, 0, 0);
                 }
             if (j > 0) add_t(j - 1);
@@ -1066,10 +1086,10 @@ __global__ __launch_bounds__(T::THREADS, 2) void split_gemm_kernel(SplitGemm g, 
             // 570 us against the compiler's order.
             if constexpr (SPREAD) {
 #pragma unroll
-                for (int r = 0; r < 6 * T::FM; ++r) {
+                for (int r = 0; r < PRODUCTS * T::FM; ++r) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                     if (r % T::FM == T::FM - 1 && r < 3 * T::FM) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                    if (r >= T::FM) __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                    if (r >= T::FM) __builtin_amdgcn_sched_group_barrier(0x002, (NC == 1 ? 2 : 3), 0);
                 }
             } else if (j != J_ST) {
 #pragma unroll

@@ -65,7 +65,7 @@ def test_every_bit_of_an_operand_arrives(M, N, Kd, trans):
 def test_sums_round_once_per_stage(M, N, Kd, trans):
     # Accumulators are rounded once per 32 k: |dC| <= (K / 32 + 8) 2^-24
     # sum |a||b| -- the 8 for the 6 MFMAs of a stage, the dropped products
-    # (2^-25 each) and the adds of k groups and splits (at most 32 more terms,
+    # (2^-24 (1 + 2^-9) together) and the adds of k groups and splits (at most 32 more terms,
     # each a partial sum of its own K range, counted in K / 32).
     print(f"split real {M}x{N}x{Kd}", flush=True)
     rng = np.random.default_rng(M * 3 + Kd)
@@ -106,6 +106,30 @@ def test_operands_outside_the_exact_range(M, N, Kd, trans):
     ref = big.astype(np.float64) @ small.astype(np.float64)
     lim = 1e-5 * np.sqrt(Kd) * (np.abs(big.astype(np.float64)) @ np.abs(small.astype(np.float64)))
     assert np.all(np.abs(got - ref) <= lim)
+
+
+def ulps(got, exact):
+    return np.abs(got - exact) / np.spacing(np.abs(exact).astype(F)).astype(np.float64)
+
+
+@pytest.mark.parametrize("M,N,Kd,trans", SHAPES)
+def test_sums_of_one_term(M, N, Kd, trans):
+    # One product per output.  Of x, y in [1, 2): |mid| <= 2^-8, |lo| <= 2^-17, so
+    # the three dropped part products are at most 2^-24 (1 + 2^-9), half a unit
+    # of the last place; the sum's cut to 24 bits is one unit, or half a unit
+    # where hi hi is added rounded (64x64 tiles); the cuts of the five small
+    # products, whose sum is below 2^-6, are 5 2^-30 2^(23) = 0.04 units.
+    print(f"split one term {M}x{N}x{Kd}", flush=True)
+    rng = np.random.default_rng(M + 3 * N)
+    pick = rng.integers(0, Kd, N)
+    a = rng.uniform(-2, 2, (M, Kd)).astype(F)
+    b = np.zeros((Kd, N), F)
+    w = b[pick, np.arange(N)] = rng.uniform(-2, 2, N).astype(F)
+    got = run(a, b, None, 0, trans)
+    err = ulps(got, a[:, pick].astype(np.float64) * w.astype(np.float64))
+    tiles64 = (M, N, Kd, trans) in SHAPES[6:]
+    print(f"largest error {err.max():.3f} units of the last place", flush=True)
+    assert err.max() <= (1.05 if tiles64 else 1.55)
 
 
 @pytest.mark.parametrize("M,N,Kd,trans", SHAPES)
@@ -330,3 +354,22 @@ def test_conv_pair_equals_its_calls_on_tiny_values(tiny):
     want = _pair_unfused(x, w1, None, w2, None, 0, 0)
     assert want.any()
     np.testing.assert_array_equal(_pair_fused(x, w1, None, w2, None, 0, 0), want)
+
+
+@pytest.mark.parametrize("geom", CONVS)
+def test_conv_sums_of_one_term(geom):
+    # As test_sums_of_one_term: a kernel of one tap of one channel, a weight of
+    # its own per output channel.
+    N, C, H_, W_, Co, KH, KW, st, pad = geom
+    print(f"split conv one term {geom}", flush=True)
+    rng = np.random.default_rng(C + 5 * Co)
+    x = rng.uniform(-2, 2, (N, C, H_, W_)).astype(F)
+    w = np.zeros((Co, C, KH, KW), F)
+    one = w[:, C - 1, KH - 1, KW - 1] = rng.uniform(-2, 2, Co).astype(F)
+    got = conv(x, w, None, geom, 0)
+    OH, OW = got.shape[2:]
+    xp = np.zeros((N, H_ + 2 * pad, W_ + 2 * pad))
+    xp[:, pad:pad + H_, pad:pad + W_] = x[:, C - 1]
+    px = xp[:, KH - 1:KH + st * (OH - 1):st, KW - 1:KW + st * (OW - 1):st]
+    exact = px[:, None] * one.astype(np.float64)[None, :, None, None]
+    assert ulps(got, exact).max() <= 1.55
