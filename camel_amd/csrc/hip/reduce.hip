@@ -496,7 +496,10 @@ int camel_hip_softmax_rows(const float *x, float *y, int64_t rows, int64_t cols)
     const int c = (int)cols;
     // Up to 4096 columns a wave holds a row.  Short rows share a wave once one
     // row per wave would queue (262144 x 10: 66 -> 12.6 us, x 64: 82 -> 24; 4096
-    // rows: 3.1 against 4.6, so not below 8192).  A row is spread over a
+    // rows: 3.1 against 4.6, so not below 8192), wider rows later, as fewer of them
+    // share a wave (one per wave / shared: 10240 x 64 4.8 / 4.5, 10240 x 128 5.3 /
+    // 5.7, 12288 x 128 5.6 / 5.8, 16385 x 128 7.3 / 5.8, 12288 x 256 6.8 / 7.3, 16385 x
+    // 256 8.3 / 7.9).  A row is spread over a
     // work-group where rows are too few for the chip (256 x 1024 3.5 -> 2.8 us;
     // 1024 rows: 3.9 both; 1024 x 2048 5.5 -> 4.9, 4096 rows: 11.8 against 13.1)
     // or too long for a wave: from 2048 columns on (16384 x 4096 95 -> 85 us, 3001
@@ -505,7 +508,7 @@ int camel_hip_softmax_rows(const float *x, float *y, int64_t rows, int64_t cols)
     // quads per thread beat 4 from 4096 columns on (1024 x 16384: 24.4 us against
     // 32.2 for 1024 x 4 quads and 25.5 for 256 x 16), whose work-groups of 1024
     // threads have a CU to themselves.
-    if (cols <= (vec ? 256 : 64) && rows > 8192)
+    if (cols <= (vec ? 256 : 64) && rows > 8192 + 32 * cols)
         CAMEL_RETURN_IF(launch_softmax_short<0>(x, y, rows, c, vec));
     else if (cols <= 256)
         CAMEL_RETURN_IF(launch_softmax<1>(x, y, rows, c, vec));

@@ -15,10 +15,10 @@ pytestmark = pytest.mark.gpu
 P = C.c_void_p
 F = np.float32
 
-# Short rows share a wave beyond 8192 rows (4096 columns of a row group are
-# the last chunk's remainder); work-groups of 256 x 1, 2, 4, 8 and 512, 1024 x 8
-# quads; the three-pass kernel from 32769 columns on.
-SHAPES = [(8193, c) for c in (1, 2, 3, 4, 5, 8, 10, 16, 17, 32, 33, 63, 64, 65, 128, 132, 252, 256)]
+# Short rows share a wave beyond 8192 + 32 cols rows (the last wave's rows are
+# few); work-groups of 256 x 1, 2, 4, 8 and 512, 1024 x 8 quads; the three-pass
+# kernel from 32769 columns on.
+SHAPES = [(8193 + 32 * c, c) for c in (1, 2, 3, 4, 5, 8, 10, 16, 17, 32, 33, 63, 64, 65, 128, 132, 252, 256)]
 SHAPES += [(8192, 10), (512, 513), (512, 1024), (513, 1023), (2048, 1025), (2049, 2048), (3, 2049),
            (5, 4095), (4, 4096), (7, 4097), (3, 8191), (2, 8192), (3, 8195), (2, 16384), (3, 16386),
            (2, 32767), (1, 32768), (2, 32769), (1, 70001)]
