@@ -1663,7 +1663,8 @@ int launch_thin(const float *A, const float *B, float *C, int M, int N, int K, c
 // 16 on guarded loads 1 x 4096 x 4096 took 16.7 us, 14.4 without; 17 rows 21.7,
 // 17.4.  N % 4 != 0, on 32 x 128 tiles against here: 16 x 3001 x 2047 18.4 and
 // 12.1, 7 x 1001 x 77 7.7 and 4.0, 12 x 5 x 3000 16.9 and 6.7, 32 x 8191 x 8192
-// 78.5 and 69.6.  16 aligned rows pay for the clamps: 16 x 4096 x 4096 14.70, 14.81.)
+// 78.5 and 69.6.  Shapes that are whole have a kernel without the clamps: 16 x
+// 4096 x 4096 14.80 with, 14.72 without.)
 constexpr int SK_WAVES = 8;
 constexpr int SK_COLS = 64;
 constexpr int SK_STEPS = 4;                          // 4-row MFMA steps per chunk and wave
@@ -1690,7 +1691,8 @@ __device__ __forceinline__ void skinny_store(float *C, int row, int ocol, int N,
             if (col + c >= ocol) out[c] = v[c];
 }
 
-template <int MT, int CH>
+// WHOLE: M = 16 MT rows, whole strips and whole k groups: no clamps, one loop.
+template <int MT, int CH, bool WHOLE>
 __global__ __launch_bounds__(SK_WAVES * 64) void sgemm_skinny_kernel(
     const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, int M, int N,
     int K, const float *__restrict__ bias, int flags, float *__restrict__ partial) {
@@ -1705,7 +1707,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void sgemm_skinny_kernel(
     const int n0 = strip * SK_COLS;
     const int kb0 = ks * KR;
     const int krow0 = kb0 + wave * 4 * S + q * S; // lane's first k of chunk 0
-    const int col = min(n0 + 4 * r16, N - 4);
+    const int col = WHOLE ? n0 + 4 * r16 : min(n0 + 4 * r16, N - 4);
 
     floatx4 acc[MT][4];
 #pragma unroll
@@ -1714,7 +1716,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void sgemm_skinny_kernel(
         for (int c = 0; c < 4; ++c) acc[t][c] = floatx4{0.f, 0.f, 0.f, 0.f};
     const float *arow[MT];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) arow[t] = A + (size_t)min(16 * t + r16, M - 1) * K;
+    for (int t = 0; t < MT; ++t) arow[t] = A + (size_t)(WHOLE ? 16 * t + r16 : min(16 * t + r16, M - 1)) * K;
 
     auto stream_k = [&](auto full_tag) {
         constexpr bool FULL = decltype(full_tag)::value;
@@ -1761,7 +1763,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void sgemm_skinny_kernel(
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    if (kb0 + KR <= K)
+    if (WHOLE || kb0 + KR <= K)
         stream_k(std::true_type{});
     else
         stream_k(std::false_type{});
@@ -1781,7 +1783,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void sgemm_skinny_kernel(
     if (x >= MT * 256) return;
     const int row = x >> 4, cg = x & 15;
     const int ocol = n0 + 4 * cg;
-    if (row >= M || ocol >= N) return;
+    if (!WHOLE && (row >= M || ocol >= N)) return;
     const int t = row >> 4, sl = ((row & 15) >> 2) * 16 + cg, e = row & 3;
     float v[4];
 #pragma unroll
@@ -1795,38 +1797,37 @@ __global__ __launch_bounds__(SK_WAVES * 64) void sgemm_skinny_kernel(
         skinny_store(C, row, ocol, N, v, bias, flags);
         return;
     }
-    *reinterpret_cast<float4 *>(partial + ((size_t)ks * M + row) * (4 * ((N + 3) / 4)) + ocol) =
+    *reinterpret_cast<float4 *>(partial + ((size_t)ks * M + row) * (WHOLE ? N : 4 * ((N + 3) / 4)) + ocol) =
         make_float4(v[0], v[1], v[2], v[3]);
 }
 
 // Sums the skinny kernel's k partials in ks order, then bias and relu; one
 // thread per column group of a row.  Small work-groups (SK_REDUCE_THREADS)
 // spread the few outputs over many CUs; the partials are read once, with
-// nontemporal loads, up to 8 k groups at a time.  Work-group b takes 4 rows of
-// strip b % strips: the skinny kernel's work-groups of that strip (block ids
+// nontemporal loads, up to 8 k groups at a time.  Work-group (strip, r) takes 4
+// rows of its strip: the skinny kernel's work-groups of that strip (block ids
 // strip + strips * ks) ran on the same XCD when strips % 8 == 0, so the
 // partials are read from that XCD's L2 (16 x 4096 x 4096: 15.30 -> 15.03 us
-// per call, against one thread per group in row-major order).
+// per call, against one thread per group in row-major order).  `total4`, the
+// quads of a k group, comes from the host: formed from M and N here, the
+// compiler multiplies each load's address out by lane (14.86 -> 14.80 us).
 constexpr int SK_REDUCE_THREADS = 64;
 static_assert(SK_REDUCE_THREADS == 4 * SK_COLS / 4, "a work-group is 4 rows of a strip");
 
 __global__ __launch_bounds__(SK_REDUCE_THREADS) void skinny_reduce_kernel(
     const float4 *__restrict__ partial, float *__restrict__ C, int M, int N, int nks,
-    const float *__restrict__ bias, int flags, int strips) {
+    const float *__restrict__ bias, int flags, size_t total4) {
     typedef float floatx4 __attribute__((ext_vector_type(4)));
-    const int strip = blockIdx.x % strips, rows4 = blockIdx.x / strips;
-    const int row = 4 * rows4 + threadIdx.x / (SK_COLS / 4);
-    const int ocol = strip * SK_COLS + 4 * (threadIdx.x % (SK_COLS / 4));
+    const int row = 4 * blockIdx.y + threadIdx.x / (SK_COLS / 4);
+    const int ocol = blockIdx.x * SK_COLS + 4 * (threadIdx.x % (SK_COLS / 4));
     if (row >= M || ocol >= N) return;
-    const int groups = (N + 3) / 4;
-    const size_t total4 = (size_t)M * groups, idx = (size_t)row * groups + ocol / 4;
-    const floatx4 *p4 = reinterpret_cast<const floatx4 *>(partial);
-    floatx4 y = __builtin_nontemporal_load(p4 + idx);
+    const floatx4 *p4 = reinterpret_cast<const floatx4 *>(partial) + (size_t)row * ((N + 3) / 4) + ocol / 4;
+    floatx4 y = __builtin_nontemporal_load(p4);
     for (int z0 = 1; z0 < nks; z0 += 8) {
         floatx4 p[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u)
-            if (z0 + u < nks) p[u] = __builtin_nontemporal_load(p4 + (size_t)(z0 + u) * total4 + idx);
+            if (z0 + u < nks) p[u] = __builtin_nontemporal_load(p4 + (size_t)(z0 + u) * total4);
 #pragma unroll
         for (int u = 0; u < 8; ++u)
             if (z0 + u < nks)
@@ -2284,21 +2285,23 @@ int launch_skinny(const float *A, const float *B, float *C, int M, int N, int K,
                            stream(), A, B, C, M, N, K, bias, flags, partial);
         CAMEL_RETURN_IF(check_launch("sgemm_skinny_kernel"));
         if (nks == 1) return CAMEL_HIP_OK;
-        hipLaunchKernelGGL(skinny_reduce_kernel, dim3((unsigned)(strips * ((M + 3) / 4))),
+        hipLaunchKernelGGL(skinny_reduce_kernel, dim3((unsigned)strips, (unsigned)((M + 3) / 4)),
                            dim3(SK_REDUCE_THREADS), 0, stream(), reinterpret_cast<const float4 *>(partial),
-                           C, M, N, nks, bias, flags, strips);
+                           C, M, N, nks, bias, flags, (size_t)M * ((N + 3) / 4));
         return check_launch("skinny_reduce_kernel");
     };
-    if (mt == 1) {
-        if (ch == 8) return go(sgemm_skinny_kernel<1, 8>);
-        if (ch == 4) return go(sgemm_skinny_kernel<1, 4>);
-        if (ch == 2) return go(sgemm_skinny_kernel<1, 2>);
-        return go(sgemm_skinny_kernel<1, 1>);
-    }
-    if (ch == 8) return go(sgemm_skinny_kernel<2, 8>);
-    if (ch == 4) return go(sgemm_skinny_kernel<2, 4>);
-    if (ch == 2) return go(sgemm_skinny_kernel<2, 2>);
-    return go(sgemm_skinny_kernel<2, 1>);
+    const bool whole = M == 16 * mt && N % SK_COLS == 0 && K % (SK_CHUNK * ch) == 0;
+    auto pick = [&](auto mt_tag, auto ch_tag) {
+        constexpr int MT = decltype(mt_tag)::value, CH = decltype(ch_tag)::value;
+        return whole ? go(sgemm_skinny_kernel<MT, CH, true>) : go(sgemm_skinny_kernel<MT, CH, false>);
+    };
+    auto by_chunks = [&](auto mt_tag) {
+        if (ch == 8) return pick(mt_tag, std::integral_constant<int, 8>{});
+        if (ch == 4) return pick(mt_tag, std::integral_constant<int, 4>{});
+        if (ch == 2) return pick(mt_tag, std::integral_constant<int, 2>{});
+        return pick(mt_tag, std::integral_constant<int, 1>{});
+    };
+    return mt == 1 ? by_chunks(std::integral_constant<int, 1>{}) : by_chunks(std::integral_constant<int, 2>{});
 }
 
 // Work-groups of one kernel that fit on the chip at once (occupancy x CUs).

@@ -298,6 +298,8 @@ def test_sgemm_special_values_propagate_like_the_reference(M, N, Kd):
     (31, 1001, 777),   # rows of A and B at every alignment
     (8, 4095, 4095),   # k groups whose partials have padded rows
     (32, 2050, 8191),  # several chunks per work-group, ragged last one
+    (16, 128, 256),    # whole strips and k groups, one and two 16-row groups
+    (32, 4096, 2048),
 ])
 def test_skinny_kernel_at_every_size_and_alignment(M, N, Kd):
     # Operands whose sums are exact: equality to the bit.  Then an operand row
