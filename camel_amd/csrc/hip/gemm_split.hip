@@ -1415,7 +1415,10 @@ SplitPlan split_gemm_plan(int64_t M, int64_t N, int64_t K, bool a_trans, bool a_
     N = up(N, 64) * 64;
     double limit = 0.9 * fp32_us(M, N, K, a_trans, a_unaligned, b_unaligned, cus);
     const double out = 4.0 * M * N / 5e6;
-    auto consider = [&](SplitTile tile, int edge, int sb, auto &&estimate) {
+    // (`least`: the estimate of one step; small products, whose calls are bound by
+    // the host, end here)
+    auto consider = [&](SplitTile tile, int edge, int sb, double least, auto &&estimate) {
+        if (limit <= least) return;
         const int64_t tiles = up(M, edge) * up(N, edge);
         if (tiles > INT32_MAX / 64) return;
         for (int want : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32}) {
