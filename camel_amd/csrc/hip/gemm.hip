@@ -2843,12 +2843,7 @@ int conv2d_gather(const float *x, const float *w, const float *bias, float *y, i
     return ok();
 }
 
-// conv2d on the split-operand kernels: x in any layout (NHWC and NCHW4 with
-// C % 4 == 0 and 16-byte alignment), y NCHW, NCHW4 (flags) or pooled.
-int conv2d_split(const float *x, const float *w, const float *bias, float *y, int64_t N, int64_t C,
-                 int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW, int64_t stride,
-                 int64_t pad, int64_t OH, int64_t OW, int flags, Layout x_layout, bool pool,
-                 bool w_packed) {
+SplitConv split_geometry(int64_t C, int64_t H, int64_t W, int64_t KH, int64_t KW, int64_t stride, int64_t pad) {
     SplitConv c{};
     c.C = (int)C;
     c.H = (int)H;
@@ -2857,6 +2852,16 @@ int conv2d_split(const float *x, const float *w, const float *bias, float *y, in
     c.KW = (int)KW;
     c.stride = (int)stride;
     c.pad = (int)pad;
+    return c;
+}
+
+// conv2d on the split-operand kernels: x in any layout (NHWC and NCHW4 with
+// C % 4 == 0 and 16-byte alignment), y NCHW, NCHW4 (flags) or pooled.
+int conv2d_split(const float *x, const float *w, const float *bias, float *y, int64_t N, int64_t C,
+                 int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW, int64_t stride,
+                 int64_t pad, int64_t OH, int64_t OW, int flags, Layout x_layout, bool pool,
+                 bool w_packed) {
+    SplitConv c = split_geometry(C, H, W, KH, KW, stride, pad);
     c.P = (int)(OH * OW);
     c.OW = (int)OW;
     c.PW = (int)(OW / 2);
@@ -2953,7 +2958,8 @@ int conv2d_run(const float *x, const float *w, const float *bias, float *y, int6
         flags &= ~CAMEL_CONV_W_PACKED;
     }
     // out_flags: the epilogue flags, plus CAMEL_CONV_Y_NCHW4 for an NCHW4 out
-    const bool split = split_conv_serves(N, C, H, W, Co, KH, KW, pad);
+    const bool split = split_conv_serves(split_geometry(C, H, W, KH, KW, stride, pad), N, N * P, Co,
+                                         device_cu_count());
     auto nhwc_gemm = [&](float *out, bool pooled, int out_flags) -> int {
         if (split)
             return conv2d_split(x, w, bias, out, N, C, H, W, Co, KH, KW, stride, pad, OH, OW, out_flags, xl,

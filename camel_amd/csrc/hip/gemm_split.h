@@ -58,9 +58,9 @@ SplitPlan split_gemm_plan(int64_t M, int64_t N, int64_t K, bool a_trans, bool a_
 // Runs it on the library stream; `partial`: plan.partial_bytes of scratch.
 int split_gemm(SplitGemm g, bool a_trans, const SplitPlan &plan, float *partial);
 
-// True when split_conv serves the geometry (either layout).
-bool split_conv_serves(int64_t N, int64_t C, int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW,
-                       int64_t pad);
+// True when split_conv serves the geometry (any layout): c's C, H, W, KH, KW,
+// stride and pad, N images, `pixels` of output in all.
+bool split_conv_serves(const SplitConv &c, int64_t N, int64_t pixels, int64_t Co, int cus);
 // The kernel and K splits of a convolution and its scratch: the split weights,
 // then the partial sums.
 struct SplitConvPlan {

@@ -1432,13 +1432,13 @@ SplitPlan split_gemm_plan(int64_t M, int64_t N, int64_t K, bool a_trans, bool a_
             }
         }
     };
-    consider(SplitTile::T256, 256, T256::SB, [&](int64_t wgs, double per, bool parts, double bytes) {
+    consider(SplitTile::T256, 256, T256::SB, 8.5 + 4.1, [&](int64_t wgs, double per, bool parts, double bytes) {
         return up(wgs, cus) * (8.5 + 4.1 * per) + (parts ? 3.6 : 0.0) + 0.9 * bytes;
     });
-    consider(SplitTile::T128, 128, T128::SB, [&](int64_t wgs, double per, bool parts, double bytes) {
+    consider(SplitTile::T128, 128, T128::SB, 8.9 + 2.06, [&](int64_t wgs, double per, bool parts, double bytes) {
         return up(wgs, cus) * (8.9 + 2.06 * per) + (parts ? 3.6 : 0.0) + 0.9 * bytes + 1.1 * out;
     });
-    consider(SplitTile::T64, 64, T64::SB, [&](int64_t wgs, double per, bool parts, double bytes) {
+    consider(SplitTile::T64, 64, T64::SB, 4.4 + 0.88, [&](int64_t wgs, double per, bool parts, double bytes) {
         const double share = wgs <= cus ? 1.0 : std::max(1.6, 0.15 + (double)wgs / cus);
         return 4.4 + per * share * (0.88 + 0.18 * a_trans) + (parts ? 2.7 : 0.0) + 1.55 * bytes + 2.5 * out;
     });
@@ -1452,14 +1452,40 @@ int split_gemm(SplitGemm g, bool a_trans, const SplitPlan &plan, float *partial)
     return launch<T64>(g, a_trans, plan.splits);
 }
 
-bool split_conv_serves(int64_t N, int64_t C, int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW,
-                       int64_t pad) {
-    const int64_t C8 = (C + 7) / 8 * 8, K = C8 * KH * KW;
+// Whether the fp32 kernels run a convolution of few stages faster: up to 9 stages
+// there are no K splits here, and the split weights are a launch of their own.
+// Microseconds up to two rounds of tiles (a tile: 128 pixels by 64 channels, or
+// 128 beyond 64 channels), from 430 measured calls; the weights' reorder, which a
+// caller with packed weights saves, counts half.  fp32 / split, packed weights:
+// 64 -> 64 1x1 at 8 x 28 x 28 7.2 / 11.1, 32 -> 64 3x3 at 8 x 28 x 28 16.9 / 20.4; and
+// unpacked 10 -> 40 3x3 at 8 x 60 x 60 14.9 / 16.4, 16 -> 32 3x3 17.3 / 16.0.  Up to
+// 16 channels the two differ by less than 10% either way, and beyond 64 the
+// fp32 tiles of few pixels take longer (128 -> 128 1x1 at 196 pixels 22.9 /
+// 17.5) but for 2 stages: those stay split, and so do geometries of the patch
+// kernel's order and of the fused pair.
+static bool fp32_conv_faster(const SplitConv &c, int64_t pixels, int64_t Co, int cus) {
+    const int taps = c.KH * c.KW, K = c.C * taps, stages = ((c.C + 7) / 8 * 8 * taps + BK - 1) / BK;
+    const bool small = Co <= 64, nhwc = c.C % 16 == 0;
+    if (stages > (small ? 9 : 2) || Co <= 16 || Co > 128 || (!nhwc && !small) || conv_blocked(c, pixels, Co, cus))
+        return false;
+    if (c.C == PAIR_C1 && c.KH == 3 && c.KW == 3 && c.stride == 1 && c.pad == 0 && c.W == PAIR_OW1) return false;
+    const int64_t tiles = (pixels + 127) / 128, rounds = (tiles + cus - 1) / cus;
+    if (rounds > 2) return false;
+    const double round = !nhwc ? 6.4 + 0.065 * K : small ? 2.8 + (c.C % 32 ? 0.07 : 0.0427) * K : 3.8 + 0.081 * K;
+    const double fp32 = 1.6 + round * (rounds > 1 ? (nhwc ? 1.8 : 1.45) : 1.0) + (nhwc ? 1.1 : 0.0);
+    const double split = (small ? 8.7 + 1.28 * stages : 11 + 1.65 * stages) + (c.C % 8 ? 1.2 : 0.0) +
+                         (rounds > 1 ? (2.5 + 0.27 * stages) * (small ? 1.0 : 1.5) : 0.0);
+    return fp32 < 0.97 * split;
+}
+
+bool split_conv_serves(const SplitConv &c, int64_t N, int64_t pixels, int64_t Co, int cus) {
+    const int64_t C8 = (c.C + 7) / 8 * 8, taps = (int64_t)c.KH * c.KW, K = C8 * taps;
     // 32 taps in a lane's mask; the divisions by C8 and KW and the buffer's
     // offsets (x, the reach of the first window, padded channels) stay exact;
     // channels padded by at most 1.6
-    return C >= 5 && KH * KW <= 32 && K >= 64 && K < 65536 && Co >= 16 &&
-           (N * C8 * H * W + 2 * pad * (W + 1) * C8) * 4 < (int64_t)1 << 30;
+    return c.C >= 5 && taps <= 32 && K >= 64 && K < 65536 && Co >= 16 &&
+           4.0 * ((double)N * c.H * c.W + 2.0 * c.pad * (c.W + 1.0)) * C8 < (double)(1 << 30) &&
+           !fp32_conv_faster(c, pixels, Co, cus);
 }
 
 SplitConvPlan split_conv_plan(const SplitGemm &g, const SplitConv &c, bool pool, int cus) {

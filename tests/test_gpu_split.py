@@ -222,11 +222,17 @@ CONVS = [
     (5, 13, 33, 31, 47, 5, 5, 2, 2),     # im2col loads, channels padded to 16, K splits
     (2, 100, 9, 7, 130, 1, 1, 1, 0),     # one tap, K % 32 = 8: stage below k = 0
     (1, 256, 7, 7, 96, 3, 3, 1, 1),      # many K splits of one tile of 49 pixels
-    (4, 32, 20, 18, 64, 3, 1, 1, 1),     # kernels of width 1: a tap is a row
+    (4, 32, 20, 18, 64, 3, 1, 1, 1),     # kernels of width 1: a tap is a row (few stages: fp32 kernels)
+    (4, 128, 20, 18, 64, 3, 1, 1, 1),
     (3, 40, 21, 17, 70, 2, 1, 2, 0),
     (2, 64, 15, 13, 130, 7, 1, 1, 0),
     (16, 32, 44, 40, 64, 5, 1, 1, 1),    # (patch)
-    (2, 32, 11, 25, 48, 1, 5, 1, 2),     # and of height 1
+    (2, 32, 11, 25, 48, 1, 5, 1, 2),     # and of height 1 (fp32 kernels)
+    (2, 80, 11, 25, 48, 1, 5, 1, 2),
+    (2, 64, 13, 15, 64, 1, 1, 1, 0),     # few stages and tiles: fp32 kernels, NHWC order
+    (2, 32, 21, 20, 64, 3, 3, 1, 1),
+    (1, 64, 17, 9, 100, 1, 1, 2, 0),     # beyond 64 channels
+    (1, 10, 31, 29, 40, 3, 3, 2, 1),     # gathered columns
 ]
 
 
