@@ -1,4 +1,7 @@
-// fp32 GEMM and implicit-GEMM conv2d on gfx950 MFMA.
+// fp32 GEMM and implicit-GEMM conv2d on gfx950 MFMA, and the choice between
+// these kernels and the split-operand ones (gemm_split.hip, bf16 matrix cores),
+// which take most products and convolutions beyond the smallest: plan_sgemm
+// (split_gemm_plan) and conv2d_run (split_conv_serves) decide.
 //
 // Replaces the ijk double loop of __tensor_matmul__
 // (modules/tensor/operators.cpp:757-766) and defines conv2d / dense on the
@@ -2924,13 +2927,16 @@ int conv_check(const float *x, const float *w, const float *bias, const float *y
     return CAMEL_HIP_OK;
 }
 
-// Every conv2d runs here.  The NHWC implicit GEMM serves C % 16 == 0 and
-// reads an NHWC or NCHW4 input in place; the direct kernel serves
-// C*KH*KW <= 32 and writes NHWC or NCHW4 directly; every other layout
-// combination goes through conversions into pooled scratch, so all of them
-// compute the same values.  pool: y is the 2x2 stride-2 max pool of the
-// result (from the GEMM epilogue when the NHWC GEMM serves the shape, else a
-// pool pass over a scratch result).
+// Every conv2d runs here.  C*KH*KW <= 32: the direct kernel, which writes NHWC
+// or NCHW4 directly.  Else the split kernels where split_conv_serves says so (C
+// >= 5, Co >= 16, up to 32 taps, buffers below 1 GiB, and not the layers of few
+// stages and tiles that the fp32 kernels run faster), and otherwise the fp32
+// implicit GEMM: NHWC order for C % 16 == 0, the gather table for the rest.  With
+// C % 16 == 0 and 16-byte alignment either one reads an NHWC or NCHW4 input in
+// place and pools in its epilogue; every other layout combination goes through
+// conversions into pooled scratch, so all of them compute the same values.
+// pool: y is the 2x2 stride-2 max pool of the result (else a pool pass over a
+// scratch result).
 int conv2d_run(const float *x, const float *w, const float *bias, float *y, int64_t N, int64_t C,
                int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW, int64_t stride, int64_t pad,
                int flags, bool pool) {

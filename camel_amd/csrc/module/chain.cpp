@@ -16,7 +16,7 @@ std::string stripPrefix(const std::string &name) {
     return name.rfind("tensor:", 0) == 0 ? name.substr(7) : name;
 }
 
-// The implicit GEMM of libcamel_hip reads an NCHW4 input in place when
+// libcamel_hip (fp32 or split-operand kernels) reads an NCHW4 input in place when
 // C % 16 == 0 and C*KH*KW exceeds the direct kernel's 32 (for an NCHW input
 // its transpose runs one image per grid z, so the batch stays below 65535).
 // Only then is an NCHW4 intermediate worth writing.

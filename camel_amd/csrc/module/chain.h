@@ -19,12 +19,13 @@
 //   conv2d -> conv2d that reads NCHW4 -> the first writes NCHW4
 //                                        ([N][C/4][H][W][4]) and the second
 //                                        reads it in place (no transpose)
-// A conv2d that runs as the implicit GEMM gets its weights packed once
-// per chain (camel_hip_conv2d_pack_weights) instead of once per call.
+// A conv2d whose input may come as NCHW4 gets its weights packed once per chain
+// (camel_hip_conv2d_pack_weights): the fp32 kernels, which layers of few stages
+// take, read them as they are; the split-operand kernels lay them out on every
+// call, packed or not.
 // Every group's values equal the layer-by-layer operators' bit for bit,
-// except conv2d + maxpool2d where the partial last round of a large
-// convolution may sum a pixel in another tile shape (within the conv2d
-// tolerance).
+// except conv2d + maxpool2d on the fp32 kernels, where the partial last round
+// may sum a pixel in another tile shape (within the conv2d tolerance).
 #pragma once
 
 #include "tensor_object.h"

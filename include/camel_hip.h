@@ -130,7 +130,10 @@ int camel_hip_eye(float *out, int64_t n);
 int camel_hip_arange(int64_t *out, int64_t start, int64_t step, int64_t count);
 
 /* ---- GEMM (tensor:matmul and dense) -------------------------------------- */
-/* C[M,N] = A[M,K] . B[K,N], fp32 row-major contiguous, on fp32 MFMA.
+/* C[M,N] = A[M,K] . B[K,N], fp32 row-major contiguous, on fp32 MFMA, or on the
+ * bf16 matrix cores with every operand as the exact sum of three bf16 parts:
+ * the sums' error is then below the fp32 MFMA chain's, that of a sum of one
+ * term up to 1.5 units of its last place.
  * Replaces the ijk loop of __tensor_matmul__ (operators.cpp:740-769).
  * flags: CAMEL_EPI_BIAS adds bias[N] to every row (the ones@b broadcast idiom,
  * test/run/nn/mnist.cml:18, then add), CAMEL_EPI_RELU applies x*(x>0)
@@ -187,16 +190,17 @@ int camel_hip_matmul_generic(int adt, const void *A, int bdt, const void *B, int
 
 /* ---- conv2d / pooling (no reference op; defined by composition) --------- */
 /* y[N,Co,OH,OW] = conv(x[N,C,H,W], w[Co,C,KH,KW]) (+bias[Co]) (relu), NCHW,
- * implicit GEMM on the same MFMA core.  OH = (H+2*pad-KH)/stride+1.
+ * implicit GEMM on the kernels of camel_hip_sgemm.  OH = (H+2*pad-KH)/stride+1.
  * flags may add the camel_hip_conv_layout bits (same values, other
  * addressing). */
 int camel_hip_conv2d(const float *x, const float *w, const float *bias, float *y, int64_t N,
                      int64_t C, int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW,
                      int64_t stride, int64_t pad, int flags);
-/* wp[Co,KH,KW,C] = w[Co,C,KH,KW] reordered: the weight layout the NHWC
+/* wp[Co,KH,KW,C] = w[Co,C,KH,KW] reordered: the weight layout the fp32 NHWC
  * implicit GEMM reads.  A caller that applies the same weights many times
- * packs them once and passes CAMEL_CONV_W_PACKED (no reference counterpart:
- * weight pre-packing of a layer chain). */
+ * packs them once and passes CAMEL_CONV_W_PACKED, which saves that kernel's
+ * reorder on each call; the split-operand kernels lay the weights out anew from
+ * either form.  (No reference counterpart: weight pre-packing of a layer chain.) */
 int camel_hip_conv2d_pack_weights(const float *w, float *wp, int64_t Co, int64_t C, int64_t KH,
                                   int64_t KW);
 /* y[N,Co,OH/2,OW/2] = maxpool2x2(conv2d(x) (+bias) (relu)), the
