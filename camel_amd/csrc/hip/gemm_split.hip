@@ -485,11 +485,11 @@ __device__ __forceinline__ void finish_sums(f4 (*acc)[FN], int kbeg, int kend, i
 // LDS as split chunks [part][octet][position]; all taps then multiply from it
 // with no conversion, store or barrier between them, and the next 32 channels'
 // loads are in flight meanwhile.  16 output pixels read 16 nearly always
-// consecutive positions, so the reads are free of bank conflicts.  Weights
-// come split, straight into registers, a tap ahead.
-// 64 x 64 x 56 x 56 -> 128 3x3: 286 us on the fp32 MFMA implicit GEMM, 206 with
-// the im2col loads above, 160 so (188 TFLOP/s; in-kernel 65% of the matrix
-// pipe's cycles, the rest the patch's conversion, tile ends and 3.1 rounds).
+// consecutive positions (an eighth of the LDS cycles are bank conflicts, where
+// they straddle rows).  Weights come split, straight into registers, a tap ahead.
+// 64 x 64 x 56 x 56 -> 128 3x3: 262 us on the fp32 MFMA implicit GEMM, 206 with
+// the im2col loads above, 140 so (211 TFLOP/s; the matrix pipe busy for 68% of
+// the kernel's cycles, the rest the patch's conversion, tile ends and 3.1 rounds).
 template <int FM_, int FN_, int WM_, int WN_> struct PatchTile {
     static constexpr int FM = FM_, FN = FN_, WM = WM_, WN = WN_;
     static constexpr int BM = 16 * FM * WM, BN = 16 * FN * WN;
@@ -686,9 +686,11 @@ __global__ __launch_bounds__(T::THREADS, 2) void conv_patch_kernel(SplitGemm g, 
 //     convolution of 32 channels, so the result equals the two conv calls and
 //     the pool bit for bit.
 // The 16 pixels of 16 columns, (2 py + r, 2 px + c) for r, c in 0..3, lie on 16
-// chunks that differ mod 16 at a row pitch of 28 (28 r = 0, 12, 8, 4 mod 16):
-// no bank conflicts.  CNN forward at batch 512: 119.0 us with the pair in fp32
-// MFMA (98 us of it), 78.6 us so.
+// chunks that differ mod 16 at a row pitch of 28 (28 r = 0, 12, 8, 4 mod 16), so
+// by the model of 16 lanes a clock the reads do not conflict; the conflict
+// counter reads 43% of the LDS cycles all the same, which is not explained.  CNN
+// forward at batch 512: 119.0 us with the pair in fp32 MFMA (98 us of it), 75.2 so
+// (51 us, the matrix pipe busy for 58% of its cycles).
 constexpr int PAIR_W = 28, PAIR_OW1 = PAIR_W - 2, PAIR_PW = (PAIR_OW1 - 2) / 2;
 constexpr int PAIR_BR = 4;                     // pooled rows per work-group
 constexpr int PAIR_R1 = 2 * PAIR_BR + 2;       // conv1 rows a band reads
@@ -1218,8 +1220,9 @@ __global__ __launch_bounds__(256) void split_conv_reduce_kernel(SplitGemm g, Spl
 
 // 256 x 256: 8 waves of 32 x 256.  128 x 128 and 64 x 64: 8 waves, 4 of 32 x 128
 // or 16 x 64 on each of two k groups (64 x 64 with the six products of a block
-// as two MFMA chains: 21.1 -> 20.2 us at 1024^3, 14.1 -> 14.5 at 68 x 192 x
-// 8021; four k groups of two 32 x 64 waves: 300 x 3000 x 800 18.8 -> 20.6).
+// as two MFMA chains: 21.1 -> 20.2 us at 1024^3, 14.1 -> 14.5 at 68 x 192 x 8021;
+// as three, hi hi by itself: 1500^3 66.7 -> 68.0; four k groups of two 32 x 64
+// waves: 300 x 3000 x 800 18.8 -> 20.6).
 using T256 = STile<2, 16, 8, 1, 1>;
 using T128 = STile<2, 8, 4, 1, 2>;
 using T64 = STile<1, 4, 4, 1, 2>;
@@ -1398,12 +1401,13 @@ static double fp32_us(int64_t M, int64_t N, int64_t K, bool at, bool ua, bool ub
 // Constants: least squares over 1500 measured (shape, tile, splits) (6% rms).
 // Over those shapes the choice is 1.21x the fp32 kernels and 2% behind the best
 // one.  Sizes enter as whole 64 x 64 tiles, so that a row gives the same bits
-// whether or not its tile is full.  Split / fp32, us: 4096^3 541 / 952, 1000 x 3001 x 2047 80 / 162, 1024 x
-// 1024 x 8192 transposed 96 / 193, 2048^3 90 / 132, 1500^3 61 / 80, 768^3 16 / 23,
-// 300 x 3000 x 800 18 / 27, 68 x 192 x 8021 transposed 14 / 17; and 1024^3 20.5 /
-// 20.5, 512^3 11.5 / 11.6, 256^3 8.1 / 5.0, which stay on the fp32 kernels: one
-// round of tiles whose loads are DMA, where a 64 x 64 split tile converts each
-// value 16 times over, and a classifier head joins the fp32 tile's epilogue.
+// whether or not its tile is full.  Split / fp32, us: 4096^3 540 / 952, 1000 x 3001 x
+// 2047 80 / 162, 1024 x 1024 x 8192 transposed 97 / 193, 2048^3 89 / 131, 1500^3 67 /
+// 79, 768^3 15.5 / 23.3, 300 x 3000 x 800 17.5 / 26.3, 68 x 192 x 8021 transposed 13.9 /
+// 16.8; and 1024^3 20.5 / 20.5, 512^3 11.5 / 11.6, 256^3 8.1 / 5.0, which stay on the
+// fp32 kernels: one round of tiles whose loads are DMA, where a 64 x 64 split tile
+// converts each value 16 times over, and a classifier head joins the fp32 tile's
+// epilogue.
 SplitPlan split_gemm_plan(int64_t M, int64_t N, int64_t K, bool a_trans, bool a_unaligned, bool b_unaligned,
                           int64_t lda, int64_t ldb, int cus) {
     SplitPlan best;
