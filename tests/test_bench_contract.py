@@ -56,7 +56,7 @@ def test_traffic_entry_parses_provenance():
     assert isinstance(src["kernels"], list) and len(src["kernels"]) == 2
     # template arguments keep their commas
     nbytes, src = bench._traffic_entry("conv2d")
-    assert "sgemm_kernel<Tile<128,128,32,2,2,1,true>,0,5>" in src["kernels"]
+    assert "conv_patch_kernel<PatchTile<2,8,4,1>,false,false>" in src["kernels"]
     assert bench._traffic_entry("no_such_workload") == (None, None)
 
 

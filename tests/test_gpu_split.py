@@ -1,7 +1,7 @@
 """The split-operand kernels (fp32 operands as three bf16 parts on the bf16
 matrix cores) at the sizes where they can go wrong: tile and stage remainders,
-K splits, transposed and unaligned operands, and operands outside the exact
-range of the split (tiles computed again in fp32)."""
+K splits, transposed and unaligned operands, the ends of the fp32 range, and
+sums that are not finite in the scaled range (formed again in fp32)."""
 import numpy as np
 import pytest
 
@@ -83,10 +83,10 @@ def test_sums_round_once_per_stage(M, N, Kd, trans):
 # at 715 x 6927 x 455, enough to change a bit of one sum in 4e6.)
 @pytest.mark.parametrize("M,N,Kd,trans", SHAPES[:9])
 def test_operands_outside_the_exact_range(M, N, Kd, trans):
-    # Values below 2^-100 lose their last part in bf16 and values near the
-    # fp32 maximum round to infinity there: their tiles run in fp32, to the
-    # fp32 kernels' bound.  Scaling by a power of two is exact, so a scaled A
-    # and a scaled B give the same bits.
+    # Values whose parts would leave the bf16 range unscaled, and values near the
+    # fp32 maximum, whose scaled parts do leave it and whose outputs are formed
+    # again in fp32: both to the fp32 kernels' bound.  Scaling by a power of two
+    # is exact, so a scaled A and a scaled B give the same bits.
     print(f"split range {M}x{N}x{Kd}", flush=True)
     rng = np.random.default_rng(M + 7 * Kd)
     a = rng.uniform(-1, 1, (M, Kd)).astype(F)
@@ -230,6 +230,8 @@ CONVS = [
     (4, 128, 20, 18, 64, 3, 1, 1, 1),
     (3, 40, 21, 17, 70, 2, 1, 2, 0),
     (2, 64, 15, 13, 130, 7, 1, 1, 0),
+    (2, 64, 19, 16, 130, 3, 1, 2, 1),    # strided and padded
+    (2, 64, 16, 19, 130, 1, 3, 2, 1),
     (16, 32, 44, 40, 64, 5, 1, 1, 1),    # (patch)
     (2, 32, 11, 25, 48, 1, 5, 1, 2),     # and of height 1 (fp32 kernels)
     (2, 80, 11, 25, 48, 1, 5, 1, 2),
@@ -307,7 +309,7 @@ def test_conv_layouts_pool_and_special_values(geom):
     xf = np.where(np.isfinite(x), 0, 1).astype(F)
     touched = conv(xf, np.ones_like(w), None, geom, 0) > 0
     assert np.array_equal(~np.isfinite(y), touched)
-    # values below the split's range: fp32 to the fp32 kernels' bound
+    # values whose parts would leave the bf16 range unscaled
     x = np.where(np.isfinite(x), x, 0).astype(F)
     base = conv(x, w, None, geom, 0)
     tiny = conv(x * F(2.0 ** -112), w, None, geom, 0).astype(np.float64) * 2.0 ** 112
