@@ -40,7 +40,6 @@
 
 #include <algorithm>
 #include <type_traits>
-#include <vector>
 
 namespace camel_hip {
 namespace {
@@ -130,6 +129,21 @@ struct Tile {
     static_assert((WK - 1) * BM * BN <= 2 * STAGE, "k-group reduction must fit the LDS buffers");
 };
 
+// n / d for 0 <= n < 2^31 by a multiplication: mul = floor(2^(31+L) / d) + 1
+// with L = ceil(log2 d), so that mul * d exceeds 2^(31+L) by at most 2^L and
+// the excess times n stays below 2^(31+L).  d = 1 has mul = 2^31 + 1.
+struct Divisor {
+    uint32_t mul, shift;
+};
+inline Divisor divisor(uint32_t d) {
+    uint32_t log = 0;
+    while (((uint64_t)1 << log) < d) ++log;
+    return {(uint32_t)(((uint64_t)1 << (31 + log)) / d + 1), 31 + log};
+}
+__device__ __forceinline__ int quotient(int n, Divisor d) {
+    return (int)(((uint64_t)(uint32_t)n * d.mul) >> d.shift);
+}
+
 struct GemmArgs {
     const float *A;  // [M, lda] row-major (conv: weights [Co, C*KH*KW]); transposed
                      // loaders: At [K, lda] row-major with lda >= M
@@ -137,7 +151,6 @@ struct GemmArgs {
     float *C;        // [M, ldc] row-major (conv: output y, NCHW)
     const float *bias;
     float *partial;  // split-K partials [split][tile of launch][BM * BN], or null
-    const int2 *ktab; // conv: per k {offset of (c,kh,kw) in x, kh << 16 | kw}
     int M, N, K;
     int lda, ldb, ldc;
     int k_per_split;  // multiple of BK
@@ -151,6 +164,9 @@ struct GemmArgs {
     // cqs = 4; NCHW4 ([N][C/4][H][W][4]) has pxs = 4, cqs = 4 * H * W.
     int P, OW, H, W, CHW, stride, pad;
     int Cin, KW, pxs, cqs;
+    // LOAD_CONV: k = (c * KH + kh) * KW + kw
+    int taps; // KH * KW
+    Divisor by_taps, by_kw;
     // LOAD_NHWC_POOL: columns in pool order, 4 per window of a 2x2 stride-2
     // max pool over a PH x PW grid (PP = PH * PW windows per image); C is the
     // pooled output [batch][M][PP]
@@ -552,13 +568,14 @@ __global__ __launch_bounds__(T::THREADS) void sgemm_kernel(GemmArgs g) {
                     const int gk = k0 + 4 * kq + u;
                     float v[4] = {0.f, 0.f, 0.f, 0.f};
                     if (FULL || (gk >= 0 && gk < kend)) {
-                        const int2 e = g.ktab[gk];
-                        const int kh = e.y >> 16, kw = e.y & 0xffff;
+                        const int ch = quotient(gk, g.by_taps), tap = gk - ch * g.taps;
+                        const int kh = quotient(tap, g.by_kw), kw = tap - kh * g.KW;
+                        const int off = ch * (g.H * g.W) + kh * g.W + kw;
 #pragma unroll
                         for (int c = 0; c < 4; ++c) {
                             const int ih = col_ih[c] + kh, iw = col_iw[c] + kw;
                             if ((unsigned)ih < (unsigned)g.H && (unsigned)iw < (unsigned)g.W)
-                                v[c] = g.B[(size_t)(col_base[c] + e.x)];
+                                v[c] = g.B[(size_t)(col_base[c] + off)];
                         }
                     }
                     rb[i][u] = make_float4(v[0], v[1], v[2], v[3]);
@@ -2797,43 +2814,19 @@ int conv2d_nhwc(const float *x, const float *w, const float *bias, float *y, int
     return ok();
 }
 
-// General path: im2col columns gathered from NCHW x through a k -> (c, kh, kw)
-// offset table built on the host once per geometry.
+// General path: im2col columns gathered from NCHW x; the loader divides k into
+// (c, kh, kw) itself, so a call leaves nothing behind for the next.  (A table
+// of the offsets, rewritten when the geometry changed, cost a copy and a wait:
+// layers 12 -> 33 3x3 of 31 x 31 and 6 -> 40 3x3 of 4 x 24 x 24 in turn took
+// 26 us a call, now 12.0; each by itself 15.3 -> 14.2 and 10.8 -> 10.0.)
 int conv2d_gather(const float *x, const float *w, const float *bias, float *y, int64_t N,
                   int64_t C, int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW,
                   int64_t stride, int64_t pad, int64_t OH, int64_t OW, int flags) {
     const int64_t K = C * KH * KW;
-    static std::vector<int2> host_tab;
-    static int2 *dev_tab = nullptr;
-    static int64_t tab_cap = 0;
-    static int64_t tab_key[4] = {-1, -1, -1, -1};
-    if (tab_key[0] != C || tab_key[1] != KH || tab_key[2] != KW || tab_key[3] != H * W * 65536 + W) {
-        if (K > tab_cap) {
-            if (dev_tab) {
-                CAMEL_RETURN_IF(check_hip(hipStreamSynchronize(stream()), "hipStreamSynchronize"));
-                camel_hip_free(dev_tab);
-            }
-            void *p = nullptr;
-            CAMEL_RETURN_IF(camel_hip_malloc(&p, (size_t)K * sizeof(int2)));
-            dev_tab = static_cast<int2 *>(p);
-            tab_cap = K;
-        }
-        host_tab.resize((size_t)K);
-        for (int64_t k = 0; k < K; ++k) {
-            const int64_t c = k / (KH * KW), r = k % (KH * KW), kh = r / KW, kw = r % KW;
-            host_tab[(size_t)k] = make_int2((int)(c * H * W + kh * W + kw), (int)((kh << 16) | kw));
-        }
-        CAMEL_RETURN_IF(check_hip(hipMemcpyAsync(dev_tab, host_tab.data(), (size_t)K * sizeof(int2),
-                                                 hipMemcpyHostToDevice, stream()),
-                                  "hipMemcpyAsync(conv table)"));
-        CAMEL_RETURN_IF(check_hip(hipStreamSynchronize(stream()), "hipStreamSynchronize"));
-        tab_key[0] = C;
-        tab_key[1] = KH;
-        tab_key[2] = KW;
-        tab_key[3] = H * W * 65536 + W;
-    }
     GemmArgs g = conv_args(w, x, bias, y, N, C, H, W, Co, KH, KW, stride, pad, OH, OW, flags);
-    g.ktab = dev_tab;
+    g.taps = (int)(KH * KW);
+    g.by_taps = divisor((uint32_t)(KH * KW));
+    g.by_kw = divisor((uint32_t)KW);
     const bool avec = (K % 4 == 0) && ((uintptr_t)w % 16 == 0);
     int rc;
     if (Co <= 64)
@@ -2931,7 +2924,7 @@ int conv_check(const float *x, const float *w, const float *bias, const float *y
 // or NCHW4 directly.  Else the split kernels where split_conv_serves says so (C
 // >= 5, Co >= 16, up to 32 taps, buffers below 1 GiB, and not the layers of few
 // stages and tiles that the fp32 kernels run faster), and otherwise the fp32
-// implicit GEMM: NHWC order for C % 16 == 0, the gather table for the rest.  With
+// implicit GEMM: NHWC order for C % 16 == 0, gathered columns for the rest.  With
 // C % 16 == 0 and 16-byte alignment either one reads an NHWC or NCHW4 input in
 // place and pools in its epilogue; every other layout combination goes through
 // conversions into pooled scratch, so all of them compute the same values.

@@ -2,6 +2,9 @@
 matrix cores) at the sizes where they can go wrong: tile and stage remainders,
 K splits, transposed and unaligned operands, the ends of the fp32 range, and
 sums that are not finite in the scaled range (formed again in fp32)."""
+import ctypes
+import gc
+
 import numpy as np
 import pytest
 
@@ -385,3 +388,35 @@ def test_conv_sums_of_one_term(geom):
     px = xp[:, KH - 1:KH + st * (OH - 1):st, KW - 1:KW + st * (OW - 1):st]
     exact = px[:, None] * one.astype(np.float64)[None, :, None, None]
     assert ulps(got, exact).max() <= 1.55
+
+
+GATHERED = [
+    (1, 12, 31, 33, 33, 3, 3, 2, 1),
+    (4, 6, 24, 23, 40, 3, 3, 1, 1),      # another geometry: offsets of its own
+    (2, 100, 9, 7, 40, 1, 1, 1, 0),      # one tap
+    (2, 20, 11, 13, 33, 3, 1, 1, 1),     # kernels of width and height 1
+    (2, 20, 11, 13, 33, 1, 3, 1, 0),
+    (1, 3, 20, 19, 130, 7, 7, 1, 3),     # more than 32 taps, more than 64 channels
+    (1, 4, 70, 72, 20, 61, 67, 1, 0),    # the longest sum
+]
+
+
+def test_gathered_convs_of_several_geometries_in_turn():
+    # Small layers and many-tap ones that gather their columns: exact whatever
+    # geometry ran before, and nothing of a call stays allocated after it.
+    from tests.test_gpu_exact import exact_conv, ternary
+    cases = []
+    for n, geom in enumerate(GATHERED):
+        N, C, H_, W_, Co, KH, KW, st, pad = geom
+        x = ternary(0x5300 + n, (N, C, H_, W_), 1)
+        w = ternary(0x5320 + n, (Co, C * KH * KW), 1).reshape(Co, C, KH, KW)
+        cases.append((geom, x, w, exact_conv(x, w, None, st, pad)))
+    used = ctypes.c_size_t()
+    H.call("camel_hip_pool_stats", ctypes.byref(used), None)
+    before = used.value
+    for geom, x, w, want in cases + cases[::-1] + cases:
+        print(f"gathered conv {geom}", flush=True)
+        assert_bits(conv(x, w, None, geom, 0), want, f"{geom}")
+    gc.collect()
+    H.call("camel_hip_pool_stats", ctypes.byref(used), None)
+    assert used.value == before
