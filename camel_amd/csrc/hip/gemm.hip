@@ -2817,7 +2817,7 @@ int conv2d_nhwc(const float *x, const float *w, const float *bias, float *y, int
 // General path: im2col columns gathered from NCHW x; the loader divides k into
 // (c, kh, kw) itself, so a call leaves nothing behind for the next.  (A table
 // of the offsets, rewritten when the geometry changed, cost a copy and a wait:
-// layers 12 -> 33 3x3 of 31 x 31 and 6 -> 40 3x3 of 4 x 24 x 24 in turn took
+// layers 12 -> 33 3x3 of 31 x 31 and 6 -> 24 3x3 of 4 x 40 x 40 in turn took
 // 26 us a call, now 12.0; each by itself 15.3 -> 14.2 and 10.8 -> 10.0.)
 int conv2d_gather(const float *x, const float *w, const float *bias, float *y, int64_t N,
                   int64_t C, int64_t H, int64_t W, int64_t Co, int64_t KH, int64_t KW,
